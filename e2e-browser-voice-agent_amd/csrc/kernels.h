@@ -27,7 +27,6 @@
 namespace q4 {
 
 constexpr int kRowTile = 64;        // rows per weight tile
-constexpr int kMaxChunk = 16;       // the reference's prompt chunk (MT, engine/cpu.js:46): the per-token matvec's tile
 constexpr int kMaxPass = 1024;      // tokens per device pass; results do not depend on the chunking
 
 // Device-resident step state: pos0 of the current pass, last sampled token.  Kernels read
@@ -467,16 +466,14 @@ struct Q4Mat {
   int N, nb, ng, nb8, Np;
 };
 
-// Accumulate, for the 16 rows of one wave, lane (r, j)'s partial sums of MT tokens in the
-// reference's block order: acc[m] = acc[m] + f32(p_j) * (dw * dx) for b = 0 .. nb-1
-// (kernels.c:137, 217-218).  Weights are read 16 bytes per lane (4 blocks of word j), a chunk of
-// 32 blocks ahead of the arithmetic.  Activation blocks come from `xs` (shared or global memory),
-// token m at xs + m * xstride4 (uint4 units), block b lane j at [b*4 + j].
-template <int MT>
-__device__ __forceinline__ void matvec_rows16(const Q4Mat& W, int tile, int rr, int j,
-                                              const uint4* __restrict__ xs, int xstride4, int M,
-                                              float (&acc)[MT]) {
+// Accumulate, for the 16 rows of one wave, lane (r, j)'s partial sum of one token in the
+// reference's block order: acc = acc + f32(p_j) * (dw * dx) for b = 0 .. nb-1 (kernels.c:137,
+// 217-218).  Weights are read 16 bytes per lane (4 blocks of word j), a chunk of 32 blocks ahead of
+// the arithmetic.  Activation blocks come from `xs` (shared memory), block b lane j at [b*4 + j].
+__device__ __forceinline__ float matvec_rows16(const Q4Mat& W, int tile, int rr, int j,
+                                               const uint4* __restrict__ xs) {
   constexpr int CG = 8;    // groups of 4 blocks per chunk
+  float acc = 0.0f;
   const uint4* wq = W.qs + ((size_t)tile * W.ng * 64 + rr) * 4 + j;
   const uint4* wd = W.d + (size_t)tile * W.nb8 * 64 + rr;
   const int nch = (W.ng + CG - 1) / CG;
@@ -510,15 +507,10 @@ __device__ __forceinline__ void matvec_rows16(const Q4Mat& W, int tile, int rr, 
           const uint32_t hbits = (hb & 1) ? (sh[hb >> 1] >> 16) : (sh[hb >> 1] & 0xffffu);
           const float dw = half_bits_to_float(hbits);
           const uint32_t lo = ww[k] & 0x0F0F0F0Fu, hi = (ww[k] >> 4) & 0x0F0F0F0Fu;
-#pragma unroll
-          for (int m = 0; m < MT; m++) {
-            if (m < M) {
-              const uint4 xv = xs[(size_t)m * xstride4 + b * 4 + j];
-              int p = sdot4(lo, xv.x, (int)xv.z);
-              p = sdot4(hi, xv.y, p);
-              acc[m] = acc[m] + (float)p * (dw * __uint_as_float(xv.w));
-            }
-          }
+          const uint4 xv = xs[b * 4 + j];
+          int p = sdot4(lo, xv.x, (int)xv.z);
+          p = sdot4(hi, xv.y, p);
+          acc = acc + (float)p * (dw * __uint_as_float(xv.w));
         }
       }
     }
@@ -529,6 +521,7 @@ __device__ __forceinline__ void matvec_rows16(const Q4Mat& W, int tile, int rr, 
       for (int c = 0; c < CG / 2; c++) sc[c] = sn[c];
     }
   }
+  return acc;
 }
 
 // ((acc_0 + acc_1) + acc_2) + acc_3 over the four lanes of a row (hsum, kernels.c:116-118);

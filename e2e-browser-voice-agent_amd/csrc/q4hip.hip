@@ -132,38 +132,23 @@ __global__ __launch_bounds__(256) void k_quant(const float* __restrict__ in, int
 
 enum { OP_STORE = 0, OP_BIAS = 1, OP_ADD = 2 };   // put() of kernels.c:190-194
 
-// y[m][n] (op)= W[n] . x[m] for M tokens (matmul_q4, kernels.c:200-273).  One wave = 16 rows;
-// lane (r, j) owns accumulator j of row r (matvec_rows16), then hsum4 and the epilogue of
-// put() (kernels.c:190-194).  For one token the activation blocks are staged in shared memory
-// (nb*64 bytes of dynamic shared memory); for a prefill chunk they are read from global memory.
-template <int MT, int OP>
-__global__ __launch_bounds__(64) void k_matvec(Q4Mat W, const uint4* __restrict__ xq, int xstride, int M,
-                                               float* __restrict__ y, int ldy, const float* __restrict__ bias) {
+// y (op)= W x for one token (matmul_q4, kernels.c:200-273).  One wave = 16 rows; lane (r, j) owns
+// accumulator j of row r (matvec_rows16), then hsum4 and the epilogue of put() (kernels.c:190-194).
+// The activation blocks are staged in shared memory (nb*64 bytes of dynamic shared memory).
+template <int OP>
+__global__ __launch_bounds__(64) void k_matvec(Q4Mat W, const uint4* __restrict__ xq, float* __restrict__ y,
+                                               const float* __restrict__ bias) {
   extern __shared__ uint4 xs[];
   const int lane = threadIdx.x, r = lane >> 2, j = lane & 3;
   const int wv = blockIdx.x, tile = wv >> 2, rr = ((wv & 3) << 4) + r;
   const int row = (tile << 6) + rr;
-  const uint4* src = xq;
-  if (MT == 1) {
-    for (int i = lane; i < W.nb * 4; i += 64) xs[i] = xq[i];
-    __syncthreads();
-    src = xs;
-  }
-  float acc[MT];
-#pragma unroll
-  for (int m = 0; m < MT; m++) acc[m] = 0.0f;
-  matvec_rows16<MT>(W, tile, rr, j, src, xstride * 4, M, acc);
-#pragma unroll
-  for (int m = 0; m < MT; m++) {
-    if (m < M) {
-      const float v = hsum4(acc[m]);
-      if (j == 0 && row < W.N) {
-        float* o = y + (size_t)m * ldy + row;
-        if (OP == OP_ADD) *o = *o + v;
-        else if (OP == OP_BIAS) *o = v + bias[row];
-        else *o = v;
-      }
-    }
+  for (int i = lane; i < W.nb * 4; i += 64) xs[i] = xq[i];
+  __syncthreads();
+  const float v = hsum4(matvec_rows16(W, tile, rr, j, xs));
+  if (j == 0 && row < W.N) {
+    if (OP == OP_ADD) y[row] = y[row] + v;
+    else if (OP == OP_BIAS) y[row] = v + bias[row];
+    else y[row] = v;
   }
 }
 
@@ -171,7 +156,7 @@ __global__ __launch_bounds__(64) void k_matvec(Q4Mat W, const uint4* __restrict_
 // heads): a grid-stride stream over 16-row groups.  Wave w of workgroup b takes groups 4b + w,
 // 4b + w + 4G, ... (G workgroups).  Each group's weights are loaded while the previous group's sums
 // run, and a wave's first loads are issued before the activation blocks are staged in shared memory
-// (once per workgroup), so the two latencies overlap.  The sums are those of k_matvec<1>: lane
+// (once per workgroup), so the two latencies overlap.  The sums are those of k_matvec: lane
 // (r, j) adds its terms acc = acc + f32(p) * (dw * dx) in block order (kernels.c:200-229), then
 // hsum4 across the row's four lanes.
 template <int NB>
@@ -260,7 +245,7 @@ inline unsigned stream_grid(int groups, int max_waves) {
   return (unsigned)((waves + 3) / 4);
 }
 
-// One token, matrices with many blocks per row (down: 896 x 4864): the same sums as k_matvec<1>,
+// One token, matrices with many blocks per row (down: 896 x 4864): the same sums as k_matvec,
 // with the blocks of a 16-row group spread over four waves.  Wave w forms the terms
 // f32(p_j) * (dw * dx) of block groups w, w + 4, ... (every term is independent of the others) into
 // shared memory; then wave 0 adds each lane's terms in block order, acc = acc + t, as
@@ -366,12 +351,12 @@ constexpr int kSplitMinBlocks = 64;
 constexpr int kSplitMaxBlocks = 480;
 inline size_t split_lds(int nb) { return (size_t)nb * 320; }
 
-// The widest row of a one-token projection on k_matvec<1> (rows wider than k_matvec_split takes):
+// The widest row of a one-token projection on k_matvec (rows wider than k_matvec_split takes):
 // 2048 blocks (K = 65536, the no-allocation matvec's limit), 64 bytes of activation block each in
 // shared memory.
 constexpr int kMatvec1MaxBlocks = 2048;
 
-// Raise the shared-memory limits of k_matvec_split and k_matvec<1> once per device, with that device
+// Raise the shared-memory limits of k_matvec_split and k_matvec once per device, with that device
 // current (before any graph capture: the handle and matvec constructors call it).
 void matvec_split_setup(int device) {
   static std::mutex mu;
@@ -382,9 +367,9 @@ void matvec_split_setup(int device) {
   (void)hipFuncSetAttribute((const void*)k_matvec_split<0>, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
   (void)hipFuncSetAttribute((const void*)k_matvec_split<1>, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
   (void)hipFuncSetAttribute((const void*)k_matvec_split<2>, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
-  (void)hipFuncSetAttribute((const void*)k_matvec<1, 0>, hipFuncAttributeMaxDynamicSharedMemorySize, lds1);
-  (void)hipFuncSetAttribute((const void*)k_matvec<1, 1>, hipFuncAttributeMaxDynamicSharedMemorySize, lds1);
-  (void)hipFuncSetAttribute((const void*)k_matvec<1, 2>, hipFuncAttributeMaxDynamicSharedMemorySize, lds1);
+  (void)hipFuncSetAttribute((const void*)k_matvec<0>, hipFuncAttributeMaxDynamicSharedMemorySize, lds1);
+  (void)hipFuncSetAttribute((const void*)k_matvec<1>, hipFuncAttributeMaxDynamicSharedMemorySize, lds1);
+  (void)hipFuncSetAttribute((const void*)k_matvec<2>, hipFuncAttributeMaxDynamicSharedMemorySize, lds1);
   (void)hipGetLastError();
   done |= (uint64_t)1 << device;
 }
@@ -1617,12 +1602,17 @@ int check_ready(q4hip* h) {
   return Q4HIP_OK;
 }
 
-// Kernel choice for passes of M > 8 tokens (every candidate gives the same bits):
+// Kernel choice for passes of M > 1 tokens (every candidate gives the same bits):
 //   k_gemm_sk (matrix cores, operands streamed through a shared-memory ring), one lane chain per
 //   wave (JS 4) when the matrix has too few rows to give 512 workgroups of 64 rows, else all four
 //   chains per wave (JS 1).  Measured on MI355X against the earlier matrix-core GEMM with register
 //   prefetch: 1024-token prefill 15.0 -> 10.5 ms, 32-sequence batched step 4.3 -> 3.7 ms.
-// Q4HIP_GEMM=valu keeps the matrix cores out (k_gemm_rows up to 64 tokens, else k_gemm_q4).
+//   From 2 tokens on: most of the 16-token tile is then idle, but a projection is bound by its
+//   chain of blocks, not by its columns.  The one-token kernel run over 2..8 tokens of activations
+//   in global memory took 34.3 ms for 4 steps of 7 sequences of the 0.5B shape, k_gemm_rows 8.8 ms,
+//   k_gemm_sk 6.7 ms.
+// Q4HIP_GEMM=valu keeps the matrix cores out (k_gemm_rows up to 64 tokens, else k_gemm_q4), as does a
+// row that is not whole groups of 4 blocks.
 enum { GK_ROWS2, GK_ROWS1, GK_TILED, GK_SK4, GK_SK1 };
 
 constexpr int kSkR4 = 4, kSkR1 = 4;    // ring slots of k_gemm_sk (JS 4: 43 KB, JS 1: 52.2 KB; 6 or 8 were slower)
@@ -1703,11 +1693,7 @@ void launch_matvec(hipStream_t s, const Mat& W, const uint4* xq, int xstride, in
     else if (W.nb >= kSplitMinBlocks && W.nb <= kSplitMaxBlocks)
       k_matvec_split<OP><<<grid, kSplitThreads, split_lds(W.nb), s>>>(W.view(), xq, y, bias);
     else
-      k_matvec<1, OP><<<grid, 64, (size_t)W.nb * 64, s>>>(W.view(), xq, xstride, 1, y, ldy, bias);
-    return;
-  }
-  if (M <= 8) {
-    k_matvec<kMaxChunk, OP><<<grid, 64, 0, s>>>(W.view(), xq, xstride, M, y, ldy, bias);
+      k_matvec<OP><<<grid, 64, (size_t)W.nb * 64, s>>>(W.view(), xq, y, bias);
     return;
   }
   switch (pick_gemm(W, M, xh != nullptr)) {
@@ -2291,7 +2277,7 @@ bool attn_list_ok(int H, int KVH, int HD, int ctx) {
 void enqueue_pass(q4hip* h, int M, bool want_logits) {
   const int D = h->D, F = h->F, HD = h->HD, QKV = h->QKV;
   hipStream_t s = h->stream;
-  uint4* xh = M > 8 ? h->xh : nullptr;
+  uint4* xh = M > 1 ? h->xh : nullptr;
   prof_mark(h, Q4HIP_PROF_EMBED);
   k_embed<<<M, 256, 0, s>>>(h->embd, D, h->tokens, h->st, h->x);
   if (M > 1 && h->list_attn == 1) k_pass_pos<<<(M + 255) / 256, 256, 0, s>>>(h->st, M, h->tpos);
@@ -3115,7 +3101,7 @@ void enqueue_batch_step(q4hip_batch* bt, int* out) {
   q4hip* h = bt->h;
   const int B = bt->B, D = h->D, F = h->F, HD = h->HD, QKV = h->QKV;
   hipStream_t s = h->stream;
-  uint4* xh = B > 8 ? h->xh : nullptr;
+  uint4* xh = B > 1 ? h->xh : nullptr;
   k_embed_list<<<B, 256, 0, s>>>(h->embd, D, bt->tok, h->x);
   for (int l = 0; l < h->NL; l++) {
     Layer& y = h->L[l];
