@@ -18,6 +18,7 @@
 #include <type_traits>
 #include <vector>
 
+#include "attn_head.h"
 #include "gemm_sk.h"
 #include "kernels.h"
 #include "persistent.h"
@@ -2173,6 +2174,37 @@ void launch_quant(hipStream_t s, int rows, const float* in, int ld_in, int n, co
   k_quant<MODE><<<xh && rows >= 128 ? 8 * ((rows + 7) / 8) : rows, 256, lds, s>>>(in, ld_in, n, w, eps, xq, xstride, m_first, xh, rows);
 }
 
+// Largest prompt pass, in (row, head) units, that k_attn_head takes: from there on the kernels that
+// read a K row once for all heads of a group are faster.  head_dim 64, against k_attn_rows, whole
+// passes of the 0.5B shape (14 heads) at position 0 and at 600: 48 tokens 1.44 / 1.79 against 1.53 /
+// 1.87 ms, 72 tokens 1.65 / 2.08 against 1.75 / 2.06 ms, 96 tokens 1.88 / 2.49 against 1.88 / 2.19 ms.
+// head_dim 128, against three launches, 1.5B shape (12 heads): 48 tokens 2.74 against 3.08 ms, 224
+// tokens 6.85 against 6.93 ms, 600 tokens 15.3 against 13.9 ms.  Batches of sequences share no cache
+// rows between them and take it at any size (32 sequences of 1,026 positions, 1.5B shape: 29.6 us a
+// layer against 33.0 for k_attn_scores_list and k_attn_pv_list), as does a single token (700
+// positions: 15.5 against 27.2 us).
+inline int head_max_units(int HD) { return HD == 64 ? 1024 : 3072; }
+
+// Raise k_attn_head's shared-memory limit once per device, with that device current (before any
+// graph capture; attn_list_ok calls it).
+bool attn_head_setup(int device) {
+  static std::mutex mu;
+  static uint64_t done = 0, ok = 0;
+  std::lock_guard<std::mutex> lock(mu);
+  if (device < 0 || device >= 64) return false;
+  if (!((done >> device) & 1)) {
+    bool all = true;
+    const void* fns[4] = {(const void*)k_attn_head<64, float>, (const void*)k_attn_head<64, kvhalf>,
+                          (const void*)k_attn_head<128, float>, (const void*)k_attn_head<128, kvhalf>};
+    for (const void* fn : fns)
+      all = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, kHeadMaxLds) == hipSuccess && all;
+    (void)hipGetLastError();
+    done |= (uint64_t)1 << device;
+    if (all) ok |= (uint64_t)1 << device;
+  }
+  return (ok >> device) & 1;
+}
+
 // V rows per chunk of k_attn_pv_list: 128 (34 KB of LDS for the two chunk buffers) halves the
 // chunk steps of 64 rows; 256 was slower again.
 constexpr int kPvRows = 128;
@@ -2193,6 +2225,18 @@ void launch_attn_list_t(hipStream_t s, int HD, int B, int H, int KVH, const floa
   const size_t lds = attn_pv_lds(H, KVH, ctx);
   const int Gq = H / KVH;
   int dev = 0;
+  if (xq && !pv_tiles_off() && (seq_stride != 0 || B == 1 || (!attn_rows_off() && B * H <= head_max_units(HD))) &&
+      (HD == 64 ? attn_head_lds<64>(ctx) : attn_head_lds<128>(ctx)) <= (size_t)kHeadMaxLds &&
+      hipGetDevice(&dev) == hipSuccess && attn_head_setup(dev)) {
+    const unsigned hg = attn_head_grid(B, KVH, Gq);
+    if (HD == 64)
+      k_attn_head<64, KT><<<hg, kHeadThreads, attn_head_lds<64>(ctx), s>>>(qkv, QKV, H, KVH, kc, vc, ctx, layer, pos, B,
+                                                                           seq_stride, xq, xstride, xh);
+    else
+      k_attn_head<128, KT><<<hg, kHeadThreads, attn_head_lds<128>(ctx), s>>>(qkv, QKV, H, KVH, kc, vc, ctx, layer, pos, B,
+                                                                             seq_stride, xq, xstride, xh);
+    return;
+  }
   if (seq_stride == 0 && B > 1 && !pv_tiles_off() && !attn_rows_off() && HD == 64 && Gq <= kMaxGroup &&
       attn_rows_lds(Gq, ctx) <= (size_t)kAttnRowsMaxLds &&
       (attn_rows_lds(Gq, ctx) <= 64 * 1024 || (hipGetDevice(&dev) == hipSuccess && attn_rows_setup(dev)))) {
@@ -2253,7 +2297,7 @@ void launch_attn_list(hipStream_t s, int HD, int B, int H, int KVH, const float*
 bool attn_list_ok(int H, int KVH, int HD, int ctx) {
   if (H / KVH > kMaxGroup) return false;
   int dev = 0;
-  if (hipGetDevice(&dev) == hipSuccess) (void)attn_rows_setup(dev);
+  if (hipGetDevice(&dev) == hipSuccess) (void)(attn_rows_setup(dev) && attn_head_setup(dev));
   const size_t lds = attn_pv_lds(H, KVH, ctx), slds = softmax_lds(H, KVH, ctx);
   if (lds > 160 * 1024) return false;
   if (slds > 64 * 1024 &&
