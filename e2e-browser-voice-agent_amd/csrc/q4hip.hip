@@ -20,6 +20,7 @@
 
 #include "attn_head.h"
 #include "gemm_sk.h"
+#include "gemm_tile.h"
 #include "kernels.h"
 #include "persistent.h"
 #include "q4hip.h"
@@ -1606,7 +1607,7 @@ int check_ready(q4hip* h) {
 // Kernel choice for passes of M > 1 tokens (every candidate gives the same bits):
 //   k_gemm_sk (matrix cores, operands streamed through a shared-memory ring), one lane chain per
 //   wave (JS 4) when the matrix has too few rows to give 512 workgroups of 64 rows, else all four
-//   chains per wave (JS 1).  Measured on MI355X against the earlier matrix-core GEMM with register
+//   chains per wave (JS 1); k_gemm_tile for large passes (tile_fills).  Measured on MI355X against the earlier matrix-core GEMM with register
 //   prefetch: 1024-token prefill 15.0 -> 10.5 ms, 32-sequence batched step 4.3 -> 3.7 ms.
 //   From 2 tokens on: most of the 16-token tile is then idle, but a projection is bound by its
 //   chain of blocks, not by its columns.  The one-token kernel run over 2..8 tokens of activations
@@ -1614,7 +1615,7 @@ int check_ready(q4hip* h) {
 //   k_gemm_sk 6.7 ms.
 // Q4HIP_GEMM=valu keeps the matrix cores out (k_gemm_rows up to 64 tokens, else k_gemm_q4), as does a
 // row that is not whole groups of 4 blocks.
-enum { GK_ROWS2, GK_ROWS1, GK_TILED, GK_SK4, GK_SK1 };
+enum { GK_ROWS2, GK_ROWS1, GK_TILED, GK_SK4, GK_SK1, GK_TILE };
 
 constexpr int kSkR4 = 4, kSkR1 = 4;    // ring slots of k_gemm_sk (JS 4: 43 KB, JS 1: 52.2 KB; 6 or 8 were slower)
 
@@ -1624,7 +1625,31 @@ bool sk_enabled() {
   return on;
 }
 
+// Whether k_gemm_tile (64 tokens x 32 rows) takes a projection of `wgs` workgroups.  Its time steps up
+// with every round of 256 workgroups (one, two, three on a CU: down of the 0.5B shape 47, 59 us for up
+// to 256, 512), where k_gemm_sk's grows with the tokens (34 us at 331, 76 us at 1,024), so it takes the
+// sizes that nearly fill their last round.  Measured on whole passes, all projections but gate|up
+// through it against none: 1.5B shape 1,000 tokens 22.4 / 23.3 ms, 640 15.0 / 15.4, 320 9.26 / 9.47,
+// but 512 (384 workgroups for o and down) 12.8 / 12.3; 0.5B shape 1,000 8.44 / 8.61, 768 6.86 / 6.50.
+constexpr int kTileMinTokens = 256;   // below, half of a 64-token tile may be idle
+inline bool tile_fills(int wgs) {
+  const int rounds = (wgs + 255) / 256, percent = wgs * 100 / (256 * rounds);
+  return percent >= (rounds == 1 ? 90 : rounds == 2 ? 85 : 75);
+}
+
+// Whether k_gemm_tile (64 tokens x one 32-value block) takes the fused gate|up projection of nrg blocks:
+// from about two workgroups per CU on; up to three token tiles only where the last one is more than half
+// full.  Whole passes through it / through k_gemm_sk: 0.5B shape 128 tokens 2.05 / 1.95 ms, 192 2.36 /
+// 2.48, 512 4.35 / 4.80, 1,000 7.65 / 8.61; 1.5B shape 128 4.15 / 4.21, 160 5.30 / 5.17, 192 5.83 /
+// 6.05, 1,000 20.4 / 23.3.
+inline bool tile_gu(int nrg, int M) {
+  const int nt = (M + 63) / 64;
+  return nrg * nt >= 456 && (nt > 3 || (M - 1) % 64 >= 32);
+}
+
 int pick_gemm(const Mat& W, int M, bool have_xh) {
+  if (have_xh && sk_enabled() && W.nb % 4 == 0 && M >= kTileMinTokens && tile_fills(W.Np / 32 * ((M + 63) / 64)))
+    return GK_TILE;
   if (have_xh && sk_enabled() && W.nb % 4 == 0)            // k_gemm_sk takes whole groups of 4 blocks
     return (W.Np / 64) * ((M + 15) / 16) >= 512 ? GK_SK1 : GK_SK4;
   if (M <= 64) return M >= 16 ? GK_ROWS2 : GK_ROWS1;
@@ -1649,13 +1674,28 @@ void launch_sk(hipStream_t s, const Mat& W, const uint4* xh, int xstride, int M,
       W.view(), xh, xstride, M, y, ldy, bias, by_tile);
 }
 
-// gate|up projection with the SwiGLU + quantize of its output fused (k_gemm_sk, EPI 1): act of the M
+// k_gemm_tile over nrg row groups.
+template <int OP, int CS, int EPI>
+void launch_tile(hipStream_t s, const Mat& W, int nrg, const uint4* xh, int xstride, int M, float* y, int ldy,
+                 const float* bias, uint4* xq_out = nullptr, uint4* xh_out = nullptr, int F = 0,
+                 const SkRope& rp = SkRope()) {
+  const int nt = (M + 63) / 64;
+  const bool by_tile = sk_by_tile(W, nt);
+  k_gemm_tile<OP, CS, EPI><<<(unsigned)sk_grid(nrg, nt, by_tile), 256, 0, s>>>(W.view(), xh, xstride, M, y, ldy, bias,
+                                                                               by_tile, xq_out, xh_out, F, rp);
+}
+
+// gate|up projection with the SwiGLU + quantize of its output fused (EPI 1): act of the M
 // tokens into xq and xh_out, exactly what the projection followed by k_quant<QM_SWIGLU> writes.
 // xh_out must not be xh_in (other workgroups still read their input blocks).  False (nothing
 // launched) where that path does not apply; the caller then runs the two launches.
 bool launch_gu_swiglu(hipStream_t s, const Mat& W, const uint4* xh_in, int xstride, int M, uint4* xq_out,
                       uint4* xh_out, int F) {
   if (!xh_in || F % 32 || !sk_enabled() || W.nb % 4) return false;
+  if (tile_gu(F / 32, M)) {
+    launch_tile<OP_STORE, 1, 1>(s, W, F / 32, xh_in, xstride, M, nullptr, 0, nullptr, xq_out, xh_out, F);
+    return true;
+  }
   const int nt = (M + 15) / 16;
   const bool by_tile = sk_by_tile(W, nt);
   k_gemm_sk<OP_STORE, 1, kSkR1, 1><<<(unsigned)sk_grid(F / 32, nt, by_tile), 256, 0, s>>>(
@@ -1663,12 +1703,18 @@ bool launch_gu_swiglu(hipStream_t s, const Mat& W, const uint4* xh_in, int xstri
   return true;
 }
 
-// q|k|v projection of a batch step with RoPE and the cache append fused (k_gemm_sk, EPI 2): q of the
-// B tokens into qkv, k and v into each sequence's cache at its position -- what the bias projection
-// followed by k_rope_kv_list writes.  False (nothing launched) where that path does not apply.
+// q|k|v projection with RoPE and the cache append fused (EPI 2): q of the M tokens into qkv, k and v
+// into the cache (of the token's sequence) at its position -- what the bias projection followed by
+// k_rope_kv or k_rope_kv_list writes.  False (nothing launched) where that path does not apply.
 bool launch_qkv_rope(hipStream_t s, const Mat& W, const uint4* xh, int xstride, int M, float* qkv, int QKV,
                      const float* bias, const SkRope& rp) {
-  if (!xh || rp.hd % 16 || pick_gemm(W, M, true) != GK_SK4) return false;
+  if (!xh || rp.hd % 32) return false;
+  const int kind = pick_gemm(W, M, true);
+  if (kind == GK_TILE) {
+    launch_tile<OP_BIAS, 2, 2>(s, W, W.Np / 32, xh, xstride, M, qkv, QKV, bias, nullptr, nullptr, 0, rp);
+    return true;
+  }
+  if (kind != GK_SK4) return false;
   const int nt = (M + 15) / 16;
   const bool by_tile = sk_by_tile(W, nt);
   k_gemm_sk<OP_BIAS, 4, kSkR4, 2><<<(unsigned)sk_grid(W.Np / 16, nt, by_tile), 256, 0, s>>>(
@@ -1700,6 +1746,7 @@ void launch_matvec(hipStream_t s, const Mat& W, const uint4* xq, int xstride, in
   switch (pick_gemm(W, M, xh != nullptr)) {
     case GK_ROWS2: launch_rows<OP, 2>(s, W, xq, xstride, M, y, ldy, bias); break;
     case GK_ROWS1: launch_rows<OP, 1>(s, W, xq, xstride, M, y, ldy, bias); break;
+    case GK_TILE: launch_tile<OP, 2, 0>(s, W, W.Np / 32, xh, xstride, M, y, ldy, bias); break;
     case GK_SK4: launch_sk<OP, 4, kSkR4>(s, W, xh, xstride, M, y, ldy, bias); break;
     case GK_SK1: launch_sk<OP, 1, kSkR1>(s, W, xh, xstride, M, y, ldy, bias); break;
     default:
@@ -2331,14 +2378,19 @@ void enqueue_pass(q4hip* h, int M, bool want_logits) {
     prof_mark(h, Q4HIP_PROF_NORM_Q);
     launch_quant<QM_NORM>(s, M, h->x, D, D, y.attn_norm, h->eps, h->xq, h->xstride, 0, xh);
     prof_mark(h, Q4HIP_PROF_QKV);
-    launch_matvec<OP_BIAS>(s, y.qkv, h->xq, h->xstride, M, h->qkv, QKV, y.bqkv, xh);
-    prof_mark(h, Q4HIP_PROF_ROPE);
-    if (h->kv16)
-      k_rope_kv<kvhalf><<<dim3(h->H + h->KVH, M), HD / 2, 0, s>>>(h->qkv, QKV, D, h->H, h->KVH, HD, h->rope, (kvhalf*)h->kc,
-                                                                  (kvhalf*)h->vc, h->ctx, l, h->st);
-    else
-      k_rope_kv<float><<<dim3(h->H + h->KVH, M), HD / 2, 0, s>>>(h->qkv, QKV, D, h->H, h->KVH, HD, h->rope, (float*)h->kc,
-                                                                 (float*)h->vc, h->ctx, l, h->st);
+    SkRope rp;
+    rp.rope = h->rope; rp.kc = h->kc; rp.vc = h->vc; rp.pos = h->tpos;
+    rp.ctx = h->ctx; rp.layer = l; rp.H = h->H; rp.KVH = h->KVH; rp.hd = HD; rp.kv16 = h->kv16;
+    if (M == 1 || h->list_attn != 1 || !launch_qkv_rope(s, y.qkv, xh, h->xstride, M, h->qkv, QKV, y.bqkv, rp)) {
+      launch_matvec<OP_BIAS>(s, y.qkv, h->xq, h->xstride, M, h->qkv, QKV, y.bqkv, xh);
+      prof_mark(h, Q4HIP_PROF_ROPE);
+      if (h->kv16)
+        k_rope_kv<kvhalf><<<dim3(h->H + h->KVH, M), HD / 2, 0, s>>>(h->qkv, QKV, D, h->H, h->KVH, HD, h->rope,
+                                                                    (kvhalf*)h->kc, (kvhalf*)h->vc, h->ctx, l, h->st);
+      else
+        k_rope_kv<float><<<dim3(h->H + h->KVH, M), HD / 2, 0, s>>>(h->qkv, QKV, D, h->H, h->KVH, HD, h->rope,
+                                                                   (float*)h->kc, (float*)h->vc, h->ctx, l, h->st);
+    }
     prof_mark(h, Q4HIP_PROF_ATTN);
     bool quantized = false;                 // the list P.V kernel wrote xq (and xh) itself
     if (M > 1 && h->ascr && h->list_attn == 1) {
