@@ -134,17 +134,30 @@ __global__ __launch_bounds__(256) void k_quant(const float* __restrict__ in, int
 
 enum { OP_STORE = 0, OP_BIAS = 1, OP_ADD = 2 };   // put() of kernels.c:190-194
 
+// The nb activation blocks of one token into shared memory: copied, or (an fp32 activation) quantized
+// as k_quant<QM_PLAIN> does.  Every workgroup of a one-token projection quantizes the whole vector
+// for itself while its first weights load: 896 values are one work item for half the threads, less
+// than the launch of its own that it replaces (a call of the 896 x 896 matvec 6.8 -> 4.5 us).
+__device__ __forceinline__ void stage_blocks(const uint4* __restrict__ xq, int nb, uint4* xs, int tid, int nthreads) {
+  for (int i = tid; i < nb * 4; i += nthreads) xs[i] = xq[i];
+}
+__device__ __forceinline__ void stage_blocks(const float* __restrict__ x, int nb, uint4* xs, int tid, int nthreads) {
+  const float none[8] = {};
+  quantize_row_dev<QM_PLAIN>(x, nullptr, 0, nb * 32, nullptr, 0.0f, xs, tid, nthreads, nullptr, 0, none, false);
+}
+
 // y (op)= W x for one token (matmul_q4, kernels.c:200-273).  One wave = 16 rows; lane (r, j) owns
 // accumulator j of row r (matvec_rows16), then hsum4 and the epilogue of put() (kernels.c:190-194).
-// The activation blocks are staged in shared memory (nb*64 bytes of dynamic shared memory).
-template <int OP>
-__global__ __launch_bounds__(64) void k_matvec(Q4Mat W, const uint4* __restrict__ xq, float* __restrict__ y,
+// The activation blocks are staged in shared memory (nb*64 bytes of dynamic shared memory).  XT: the
+// activation as given, in blocks (uint4) or in fp32 (stage_blocks).
+template <int OP, class XT>
+__global__ __launch_bounds__(64) void k_matvec(Q4Mat W, const XT* __restrict__ x, float* __restrict__ y,
                                                const float* __restrict__ bias) {
   extern __shared__ uint4 xs[];
   const int lane = threadIdx.x, r = lane >> 2, j = lane & 3;
   const int wv = blockIdx.x, tile = wv >> 2, rr = ((wv & 3) << 4) + r;
   const int row = (tile << 6) + rr;
-  for (int i = lane; i < W.nb * 4; i += 64) xs[i] = xq[i];
+  stage_blocks(x, W.nb, xs, lane, 64);
   __syncthreads();
   const float v = hsum4(matvec_rows16(W, tile, rr, j, xs));
   if (j == 0 && row < W.N) {
@@ -213,8 +226,8 @@ __device__ __forceinline__ void stream_rows(const Q4Mat& W, int g16, int r, int 
   }
 }
 
-template <int NB, int OP>
-__global__ __launch_bounds__(256) void k_matvec_stream(Q4Mat W, const uint4* __restrict__ xq, float* __restrict__ y,
+template <int NB, int OP, class XT>
+__global__ __launch_bounds__(256) void k_matvec_stream(Q4Mat W, const XT* __restrict__ x, float* __restrict__ y,
                                                       const float* __restrict__ bias) {
   __shared__ uint4 xs[NB * 4];
   const int tid = threadIdx.x, lane = tid & 63, r = lane >> 2, j = lane & 3;
@@ -222,7 +235,7 @@ __global__ __launch_bounds__(256) void k_matvec_stream(Q4Mat W, const uint4* __r
   int g16 = (int)blockIdx.x * 4 + (tid >> 6);
   StreamRegs<NB> ra, rb;
   if (g16 < groups) stream_issue<NB>(W, g16, r, j, ra);
-  for (int i = tid; i < NB * 4; i += 256) xs[i] = xq[i];
+  stage_blocks(x, NB, xs, tid, 256);
   lds_barrier();
   // two register sets, alternating, so that neither is indexed at run time
   while (g16 < groups) {
@@ -254,15 +267,15 @@ inline unsigned stream_grid(int groups, int max_waves) {
 // matvec_rows16 does (kernels.c:200-229), and the four lanes of a row combine in hsum order.
 // Dynamic shared memory: nb * 64 bytes of activation blocks, then nb * 256 bytes of terms.
 constexpr int kSplitWaves = 8, kSplitThreads = 64 * kSplitWaves;
-template <int OP>
-__global__ __launch_bounds__(kSplitThreads) void k_matvec_split(Q4Mat W, const uint4* __restrict__ xq, float* __restrict__ y,
+template <int OP, class XT>
+__global__ __launch_bounds__(kSplitThreads) void k_matvec_split(Q4Mat W, const XT* __restrict__ x, float* __restrict__ y,
                                                      const float* __restrict__ bias) {
   extern __shared__ uint4 xs[];
   float* tm = reinterpret_cast<float*>(xs + W.nb * 4);     // [block][lane (r, j)]
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, r = lane >> 2, j = lane & 3;
   const int wv = blockIdx.x, tile = wv >> 2, rr = ((wv & 3) << 4) + r;
   const int row = (tile << 6) + rr;
-  for (int i = tid; i < W.nb * 4; i += kSplitThreads) xs[i] = xq[i];
+  stage_blocks(x, W.nb, xs, tid, kSplitThreads);
   const uint4* wq = W.qs + ((size_t)tile * W.ng * 64 + rr) * 4 + j;
   const uint4* wd = W.d + (size_t)tile * W.nb8 * 64 + rr;
   constexpr int CG = 8;                                     // this wave's groups in flight
@@ -366,12 +379,11 @@ void matvec_split_setup(int device) {
   std::lock_guard<std::mutex> lock(mu);
   if (device < 0 || device >= 64 || (done >> device) & 1) return;
   const int lds = (int)split_lds(kSplitMaxBlocks), lds1 = kMatvec1MaxBlocks * 64;
-  (void)hipFuncSetAttribute((const void*)k_matvec_split<0>, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
-  (void)hipFuncSetAttribute((const void*)k_matvec_split<1>, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
-  (void)hipFuncSetAttribute((const void*)k_matvec_split<2>, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
-  (void)hipFuncSetAttribute((const void*)k_matvec<0>, hipFuncAttributeMaxDynamicSharedMemorySize, lds1);
-  (void)hipFuncSetAttribute((const void*)k_matvec<1>, hipFuncAttributeMaxDynamicSharedMemorySize, lds1);
-  (void)hipFuncSetAttribute((const void*)k_matvec<2>, hipFuncAttributeMaxDynamicSharedMemorySize, lds1);
+  const void* split[4] = {(const void*)k_matvec_split<0, uint4>, (const void*)k_matvec_split<1, uint4>,
+                          (const void*)k_matvec_split<2, uint4>, (const void*)k_matvec_split<0, float>};
+  const void* one[3] = {(const void*)k_matvec<0, uint4>, (const void*)k_matvec<1, uint4>, (const void*)k_matvec<2, uint4>};
+  for (const void* fn : split) (void)hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+  for (const void* fn : one) (void)hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, lds1);
   (void)hipGetLastError();
   done |= (uint64_t)1 << device;
 }
@@ -1728,21 +1740,25 @@ void launch_rows(hipStream_t s, const Mat& W, const uint4* xq, int xstride, int 
       W.view(), xq, xstride, M, y, ldy, bias);
 }
 
+// One token: xq its activation blocks, or (XT float) the activation itself, rows of up to
+// kSplitMaxBlocks blocks.
+template <int OP, class XT>
+void launch_matvec1(hipStream_t s, const Mat& W, const XT* x, float* y, const float* bias) {
+  const unsigned grid = (unsigned)(W.Np / 16);
+  if (W.nb == 28)
+    k_matvec_stream<28, OP, XT><<<stream_grid(W.Np / 16, stream_waves(28)), 256, 0, s>>>(W.view(), x, y, bias);
+  else if (W.nb == 48)
+    k_matvec_stream<48, OP, XT><<<stream_grid(W.Np / 16, stream_waves(48)), 256, 0, s>>>(W.view(), x, y, bias);
+  else if (W.nb >= kSplitMinBlocks && W.nb <= kSplitMaxBlocks)
+    k_matvec_split<OP, XT><<<grid, kSplitThreads, split_lds(W.nb), s>>>(W.view(), x, y, bias);
+  else
+    k_matvec<OP, XT><<<grid, 64, (size_t)W.nb * 64, s>>>(W.view(), x, y, bias);
+}
+
 template <int OP>
 void launch_matvec(hipStream_t s, const Mat& W, const uint4* xq, int xstride, int M, float* y, int ldy,
                    const float* bias, const uint4* xh = nullptr) {
-  const unsigned grid = (unsigned)(W.Np / 16);
-  if (M == 1) {
-    if (W.nb == 28)
-      k_matvec_stream<28, OP><<<stream_grid(W.Np / 16, stream_waves(28)), 256, 0, s>>>(W.view(), xq, y, bias);
-    else if (W.nb == 48)
-      k_matvec_stream<48, OP><<<stream_grid(W.Np / 16, stream_waves(48)), 256, 0, s>>>(W.view(), xq, y, bias);
-    else if (W.nb >= kSplitMinBlocks && W.nb <= kSplitMaxBlocks)
-      k_matvec_split<OP><<<grid, kSplitThreads, split_lds(W.nb), s>>>(W.view(), xq, y, bias);
-    else
-      k_matvec<OP><<<grid, 64, (size_t)W.nb * 64, s>>>(W.view(), xq, y, bias);
-    return;
-  }
+  if (M == 1) return launch_matvec1<OP>(s, W, xq, y, bias);
   switch (pick_gemm(W, M, xh != nullptr)) {
     case GK_ROWS2: launch_rows<OP, 2>(s, W, xq, xstride, M, y, ldy, bias); break;
     case GK_ROWS1: launch_rows<OP, 1>(s, W, xq, xstride, M, y, ldy, bias); break;
@@ -3593,14 +3609,21 @@ int q4hip_mv_run_noalloc(q4hip_mv* m, const float* x, float* y, void* stream) {
   if (K > Q4HIP_NOALLOC_MAX_K)
     return fail(Q4HIP_EINVAL, "K = %d exceeds the no-allocation limit of %d", K, Q4HIP_NOALLOC_MAX_K);
   HIPCHK(hipSetDevice(m->device));
+  // x is quantized once, in a launch of its own, for rows past kSplitMaxBlocks and where y overlaps it
+  // (a workgroup's results would change what a later one reads)
+  const bool fused = m->W.nb <= kSplitMaxBlocks && (y >= x + K || x >= y + N);
   uint4* xq = nullptr;
-  int rc = scratch_on(m->device, &xq);
+  int rc = fused ? Q4HIP_OK : scratch_on(m->device, &xq);
   if (rc == Q4HIP_OK) rc = check_device_span(x, (size_t)K * 4, m->device, "x");
   if (rc == Q4HIP_OK) rc = check_device_span(y, (size_t)N * 4, m->device, "y");
   if (rc != Q4HIP_OK) return rc;
   hipStream_t s = stream ? (hipStream_t)stream : m->stream;
-  launch_quant<QM_PLAIN>(s, 1, x, K, K, nullptr, 0.0f, xq, K / 32, 0);
-  launch_matvec<OP_STORE>(s, m->W, xq, m->W.nb, 1, y, N, nullptr);
+  if (fused) {
+    launch_matvec1<OP_STORE>(s, m->W, x, y, nullptr);
+  } else {
+    launch_quant<QM_PLAIN>(s, 1, x, K, K, nullptr, 0.0f, xq, K / 32, 0);
+    launch_matvec<OP_STORE>(s, m->W, xq, m->W.nb, 1, y, N, nullptr);
+  }
   HIPCHK(hipGetLastError());
   if (!stream) HIPCHK(hipStreamSynchronize(s));
   return Q4HIP_OK;
