@@ -191,10 +191,9 @@ __device__ __forceinline__ void stream_issue(const Q4Mat& W, int g16, int r, int
   for (int c = 0; c < StreamRegs<NB>::NS; c++) R.s[c] = wd[(size_t)c * 64];
 }
 
-template <int NB, int OP>
-__device__ __forceinline__ void stream_rows(const Q4Mat& W, int g16, int r, int j, const uint4* xs,
-                                            const StreamRegs<NB>& R, float* __restrict__ y,
-                                            const float* __restrict__ bias) {
+// The dot product of this lane's row (in every lane of its quad).
+template <int NB>
+__device__ __forceinline__ float stream_dot(int j, const uint4* xs, const StreamRegs<NB>& R) {
   float acc = 0.0f;
 #pragma unroll
   for (int g = 0; g < StreamRegs<NB>::NG; g++) {
@@ -216,8 +215,15 @@ __device__ __forceinline__ void stream_rows(const Q4Mat& W, int g16, int r, int 
       }
     }
   }
-  const float v = hsum4(acc);
-  const int row = ((g16 >> 2) << 6) + ((g16 & 3) << 4) + r;
+  return hsum4(acc);
+}
+
+template <int NB, int OP>
+__device__ __forceinline__ void stream_rows(const Q4Mat& W, int g16, int r, int j, const uint4* xs,
+                                            const StreamRegs<NB>& R, float* __restrict__ y,
+                                            const float* __restrict__ bias) {
+  const float v = stream_dot<NB>(j, xs, R);
+  const int row = (g16 << 4) + r;
   if (j == 0 && row < W.N) {
     float* o = y + row;
     if (OP == OP_ADD) *o = *o + v;
@@ -247,6 +253,90 @@ __global__ __launch_bounds__(256) void k_matvec_stream(Q4Mat W, const XT* __rest
     if (g2 < groups) stream_issue<NB>(W, g2, r, j, ra);
     stream_rows<NB, OP>(W, g1, r, j, xs, rb, y, bias);
     g16 = g2;
+  }
+}
+
+// One token, rows of NB blocks: RMSNorm + quantize of x, the q|k|v or gate|up projection and what follows
+// it, in one launch (the chain RMSNorm, projection, RoPE or SwiGLU took three).  These steps are latency,
+// not work: a launch costs more than forming the 896 or 1536 normalised values again in every
+// workgroup, and a wave's weights load meanwhile.  Each wave takes one 16-row group, placed so that what
+// the epilogue combines meets in a workgroup:
+//   EPI 1  gate|up of ffn rows each: waves 0, 1 the gate rows of one 32-value block, waves 2, 3 its up
+//          rows; SwiGLU and quantize of the block into xq_out (k_quant<QM_SWIGLU>'s block)
+//   EPI 2  q|k|v: wave w and wave w ^ 2 hold the two halves of 16 RoPE pairs of a head; bias, RoPE at
+//          st->pos0, q to y, k and v to the cache (what k_rope_kv writes)
+// The 1.5B shape at 700 positions, per layer: RMSNorm 4.8 + q|k|v 5.7 + RoPE 2.8 us -> 7.4 us; RMSNorm
+// 4.8 + gate|up 8.7 + SwiGLU 7.8 -> 10.6 us.
+template <int NB, int EPI, class KT>
+__global__ __launch_bounds__(256) void k_token_proj(Q4Mat W, const float* __restrict__ x, const float* __restrict__ w,
+                                                   float eps, uint4* __restrict__ xq_out, int ffn,
+                                                   float* __restrict__ y, const float* __restrict__ bias,
+                                                   const float* __restrict__ rope, KT* __restrict__ kc,
+                                                   KT* __restrict__ vc, int H, int KVH, int hd, int ctx, int layer,
+                                                   const State* __restrict__ st_) {
+  constexpr int n = NB * 32, sst = ((n / 4 + 31) & ~31) + 32, st = n / 4 + 1;      // sst = sq_stride(n)
+  __shared__ __align__(16) float sq[4 * sst];
+  __shared__ float xl[4 * st], red[4], ex[4][16];
+  __shared__ uint4 xs[NB * 4];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, r = lane >> 2, j = lane & 3, b = blockIdx.x;
+  int g16;
+  if (EPI == 1) {
+    g16 = (wave < 2 ? 0 : ffn >> 4) + 2 * b + (wave & 1);
+  } else {
+    const int gph = hd >> 4, wph = gph >> 2, head = b / wph;       // 16-row groups, workgroups of a head
+    g16 = head * gph + 2 * (b - head * wph) + (wave & 1) + (wave >> 1) * (gph >> 1);
+  }
+  StreamRegs<NB> R;
+  stream_issue<NB>(W, g16, r, j, R);
+  float wv[8];
+  const bool one = tid < NB * 4;                             // at most one work item per thread
+  static_assert(NB * 4 <= 256, "one quantize work item per thread");
+  if (one) norm_weights_item(w, tid, wv);
+  sq_stage(x, n, sq, sst, xl, st, tid, 256);
+  lds_barrier();
+  if (tid < 4) red[tid] = ordered_sum(sq + tid * sst, n >> 2);
+  lds_barrier();
+  const float ss = red[0] + red[1] + red[2] + red[3];
+  const float rs = 1.0f / __builtin_sqrtf(ss / (float)n + eps);
+  quantize_row_dev<QM_NORM>(nullptr, xl, st, n, w, rs, xs, tid, 256, nullptr, 0, wv, true);
+  lds_barrier();
+  const float v = stream_dot<NB>(j, xs, R);
+  if (EPI == 1) {
+    if (j == 0) ex[wave][r] = v;                             // [gate 0..31, up 0..31]
+    lds_barrier();
+    if (tid < 4) {
+      const float* g = ex[0];
+      float gv[8], uv[8], a[8];
+      const int e[8] = {2 * j, 2 * j + 1, 8 + 2 * j, 9 + 2 * j, 16 + 2 * j, 17 + 2 * j, 24 + 2 * j, 25 + 2 * j};
+#pragma unroll
+      for (int k = 0; k < 8; k++) {
+        gv[k] = g[e[k]];
+        uv[k] = g[32 + e[k]];
+      }
+      swiglu8(gv, uv, a);
+      quantize_item(a, b, j, xq_out, nullptr);
+    }
+  } else {
+    const int row = (g16 << 4) + r, head = row / hd, el = row - head * hd, half = hd >> 1, i = el < half ? el : el - half;
+    const float xv = v + bias[row];
+    if (j == 0) ex[wave][r] = xv;
+    lds_barrier();
+    if (j == 0) {
+      const int p = st_->pos0;
+      const float xo = ex[wave ^ 2][r];
+      float out = xv;
+      if (head < H + KVH) {
+        const float c = rope[(size_t)p * hd + 2 * i], sn = rope[(size_t)p * hd + 2 * i + 1];
+        out = el < half ? xv * c - xo * sn : xv * c + xo * sn;
+      }
+      if (head < H) {
+        y[row] = out;
+      } else {
+        const bool isv = head >= H + KVH;
+        const int kh = head - H - (isv ? KVH : 0);
+        (isv ? vc : kc)[(((size_t)layer * KVH + kh) * ctx + p) * hd + el] = (KT)out;
+      }
+    }
   }
 }
 
@@ -1771,6 +1861,28 @@ void launch_matvec(hipStream_t s, const Mat& W, const uint4* xq, int xstride, in
   }
 }
 
+// k_token_proj for the context's shape: false (nothing launched) where its rows are not 28 or 48 blocks.
+template <int EPI>
+bool launch_token_proj(hipStream_t s, q4hip* h, const Mat& W, const float* norm, int layer, const float* bias) {
+  const unsigned grid = (unsigned)(EPI == 1 ? h->F / 32 : W.N / 64);
+  auto go = [&](auto nb, auto kt) {
+    typedef decltype(kt) KT;
+    k_token_proj<decltype(nb)::value, EPI, KT><<<grid, 256, 0, s>>>(W.view(), h->x, norm, h->eps, h->xq, h->F, h->qkv, bias,
+                                                                    h->rope, (KT*)h->kc, (KT*)h->vc, h->H, h->KVH, h->HD,
+                                                                    h->ctx, layer, h->st);
+  };
+  typedef std::integral_constant<int, 28> N28;
+  typedef std::integral_constant<int, 48> N48;
+  if (W.nb == 28) {
+    if (EPI == 2 && h->kv16) go(N28(), kvhalf()); else go(N28(), float());
+  } else if (W.nb == 48) {
+    if (EPI == 2 && h->kv16) go(N48(), kvhalf()); else go(N48(), float());
+  } else {
+    return false;
+  }
+  return true;
+}
+
 // logits = head . x for one token: Q4_0 (the synthetic configurations) or Q8_0 (real files).
 void launch_head(hipStream_t s, const Mat& W, const uint4* xq, float* logits) {
   if (W.fmt == Q4HIP_TYPE_Q8_0)
@@ -2391,21 +2503,24 @@ void enqueue_pass(q4hip* h, int M, bool want_logits) {
   const size_t attn_lds = (size_t)(HD + h->ctx) * sizeof(float);
   for (int l = 0; l < h->NL; l++) {
     Layer& y = h->L[l];
-    prof_mark(h, Q4HIP_PROF_NORM_Q);
-    launch_quant<QM_NORM>(s, M, h->x, D, D, y.attn_norm, h->eps, h->xq, h->xstride, 0, xh);
     prof_mark(h, Q4HIP_PROF_QKV);
-    SkRope rp;
-    rp.rope = h->rope; rp.kc = h->kc; rp.vc = h->vc; rp.pos = h->tpos;
-    rp.ctx = h->ctx; rp.layer = l; rp.H = h->H; rp.KVH = h->KVH; rp.hd = HD; rp.kv16 = h->kv16;
-    if (M == 1 || h->list_attn != 1 || !launch_qkv_rope(s, y.qkv, xh, h->xstride, M, h->qkv, QKV, y.bqkv, rp)) {
-      launch_matvec<OP_BIAS>(s, y.qkv, h->xq, h->xstride, M, h->qkv, QKV, y.bqkv, xh);
-      prof_mark(h, Q4HIP_PROF_ROPE);
-      if (h->kv16)
-        k_rope_kv<kvhalf><<<dim3(h->H + h->KVH, M), HD / 2, 0, s>>>(h->qkv, QKV, D, h->H, h->KVH, HD, h->rope,
-                                                                    (kvhalf*)h->kc, (kvhalf*)h->vc, h->ctx, l, h->st);
-      else
-        k_rope_kv<float><<<dim3(h->H + h->KVH, M), HD / 2, 0, s>>>(h->qkv, QKV, D, h->H, h->KVH, HD, h->rope,
-                                                                   (float*)h->kc, (float*)h->vc, h->ctx, l, h->st);
+    if (M != 1 || !launch_token_proj<2>(s, h, y.qkv, y.attn_norm, l, y.bqkv)) {
+      prof_mark(h, Q4HIP_PROF_NORM_Q);
+      launch_quant<QM_NORM>(s, M, h->x, D, D, y.attn_norm, h->eps, h->xq, h->xstride, 0, xh);
+      prof_mark(h, Q4HIP_PROF_QKV);
+      SkRope rp;
+      rp.rope = h->rope; rp.kc = h->kc; rp.vc = h->vc; rp.pos = h->tpos;
+      rp.ctx = h->ctx; rp.layer = l; rp.H = h->H; rp.KVH = h->KVH; rp.hd = HD; rp.kv16 = h->kv16;
+      if (M == 1 || h->list_attn != 1 || !launch_qkv_rope(s, y.qkv, xh, h->xstride, M, h->qkv, QKV, y.bqkv, rp)) {
+        launch_matvec<OP_BIAS>(s, y.qkv, h->xq, h->xstride, M, h->qkv, QKV, y.bqkv, xh);
+        prof_mark(h, Q4HIP_PROF_ROPE);
+        if (h->kv16)
+          k_rope_kv<kvhalf><<<dim3(h->H + h->KVH, M), HD / 2, 0, s>>>(h->qkv, QKV, D, h->H, h->KVH, HD, h->rope,
+                                                                      (kvhalf*)h->kc, (kvhalf*)h->vc, h->ctx, l, h->st);
+        else
+          k_rope_kv<float><<<dim3(h->H + h->KVH, M), HD / 2, 0, s>>>(h->qkv, QKV, D, h->H, h->KVH, HD, h->rope,
+                                                                     (float*)h->kc, (float*)h->vc, h->ctx, l, h->st);
+      }
     }
     prof_mark(h, Q4HIP_PROF_ATTN);
     bool quantized = false;                 // the list P.V kernel wrote xq (and xh) itself
@@ -2448,16 +2563,19 @@ void enqueue_pass(q4hip* h, int M, bool want_logits) {
     if (!quantized) launch_quant<QM_PLAIN>(s, M, h->att, D, D, nullptr, 0.0f, h->xq, h->xstride, 0, xh);
     prof_mark(h, Q4HIP_PROF_O);
     launch_matvec<OP_ADD>(s, y.o, h->xq, h->xstride, M, h->x, D, nullptr, xh);
-    prof_mark(h, Q4HIP_PROF_NORM_Q);
-    launch_quant<QM_NORM>(s, M, h->x, D, D, y.ffn_norm, h->eps, h->xq, h->xstride, 0, xh);
-    prof_mark(h, Q4HIP_PROF_GU);
     uint4* xh_act = xh;      // where the down projection finds the activation's fp16 operands
-    if (launch_gu_swiglu(s, y.gu, xh, h->xstride, M, h->xq, h->xh2, F)) {
-      xh_act = h->xh2;
-    } else {
-      launch_matvec<OP_STORE>(s, y.gu, h->xq, h->xstride, M, h->gu, 2 * F, nullptr, xh);
-      prof_mark(h, Q4HIP_PROF_SWIGLU);
-      launch_quant<QM_SWIGLU>(s, M, h->gu, 2 * F, F, nullptr, 0.0f, h->xq, h->xstride, 0, xh);
+    prof_mark(h, Q4HIP_PROF_GU);
+    if (M != 1 || !launch_token_proj<1>(s, h, y.gu, y.ffn_norm, l, nullptr)) {
+      prof_mark(h, Q4HIP_PROF_NORM_Q);
+      launch_quant<QM_NORM>(s, M, h->x, D, D, y.ffn_norm, h->eps, h->xq, h->xstride, 0, xh);
+      prof_mark(h, Q4HIP_PROF_GU);
+      if (launch_gu_swiglu(s, y.gu, xh, h->xstride, M, h->xq, h->xh2, F)) {
+        xh_act = h->xh2;
+      } else {
+        launch_matvec<OP_STORE>(s, y.gu, h->xq, h->xstride, M, h->gu, 2 * F, nullptr, xh);
+        prof_mark(h, Q4HIP_PROF_SWIGLU);
+        launch_quant<QM_SWIGLU>(s, M, h->gu, 2 * F, F, nullptr, 0.0f, h->xq, h->xstride, 0, xh);
+      }
     }
     prof_mark(h, Q4HIP_PROF_DOWN);
     launch_matvec<OP_ADD>(s, y.down, h->xq, h->xstride, M, h->x, D, nullptr, xh_act);

@@ -2,10 +2,13 @@
 q4hip_mv_run: rows of each kernel's block counts and around its limits, ragged row counts, and y written
 over x (which takes a quantize launch of its own).  Bit for bit.
 """
+import ctypes
+
 import numpy as np
 import pytest
 
 import synth
+from test_zz_no_alloc import DevBuf, _hip
 
 pytestmark = pytest.mark.gpu
 
@@ -14,7 +17,8 @@ pytestmark = pytest.mark.gpu
                                   (129, 64), (896, 152), (48, 480), (48, 481)])
 def test_device_call_equals_run(N, nb):
     import q4hip
-    import torch
+    hip = _hip()
+    assert hip.hipSetDevice(0) == 0
     K = 32 * nb
     rng = np.random.default_rng(N + nb)
     w = synth.quantize_q4_0(rng.standard_normal(N * K, dtype=np.float32) * np.float32(0.02))
@@ -23,16 +27,23 @@ def test_device_call_equals_run(N, nb):
     print(f"{N} x {K}", flush=True)
     mv = q4hip.Matvec(w, N, K)
     want = mv.run(x)
-    s = torch.cuda.Stream()
-    buf = torch.zeros(K + N + 1, device="cuda")
-    off = 1                                     # x at 4-byte alignment only
-    buf[off:off + K] = torch.from_numpy(x).cuda()
-    y = torch.zeros(N, device="cuda")
-    torch.cuda.synchronize()
-    for _ in range(2):
-        mv.run_device(buf.data_ptr() + 4 * off, y.data_ptr(), s.cuda_stream)
-    torch.cuda.synchronize()
-    assert np.array_equal(y.cpu().numpy().view(np.uint32), want.view(np.uint32))
-    mv.run_device(buf.data_ptr() + 4 * off, buf.data_ptr() + 4 * (off + K // 2), s.cuda_stream)   # over x's second half
-    torch.cuda.synchronize()
-    assert np.array_equal(buf[off + K // 2:off + K // 2 + N].cpu().numpy().view(np.uint32), want.view(np.uint32))
+    stream = ctypes.c_void_p()
+    assert hip.hipStreamCreate(ctypes.byref(stream)) == 0
+    buf, y = DevBuf(hip, 4 * (K + N + 1)), DevBuf(hip, 4 * N)
+    try:
+        host = np.zeros(K + N + 1, np.float32)
+        host[1:1 + K] = x                       # x at 4-byte alignment only
+        buf.put(host)
+        xp = buf.p.value + 4
+        for _ in range(2):
+            mv.run_device(xp, y.p.value, stream.value)
+        assert hip.hipStreamSynchronize(stream) == 0
+        assert np.array_equal(y.get(N).view(np.uint32), want.view(np.uint32))
+        mv.run_device(xp, xp + 4 * (K // 2), stream.value)      # y over x's second half
+        assert hip.hipStreamSynchronize(stream) == 0
+        got = buf.get(K + N + 1)[1 + K // 2:1 + K // 2 + N]
+        assert np.array_equal(got.view(np.uint32), want.view(np.uint32))
+    finally:
+        buf.free()
+        y.free()
+        hip.hipStreamDestroy(stream)
