@@ -74,6 +74,16 @@ __device__ __forceinline__ void sk_dma4(const void* src, const void* lds) {
   asm volatile("s_nop 0\n\tglobal_load_lds_dword %0, off" ::"v"(src), "{m0}"(a) : "memory");
 }
 
+// The same from a wave-uniform base and a 32-bit byte offset per lane.
+__device__ __forceinline__ void sk_dma16s(const void* base, uint32_t off, const void* lds) {
+  const uint32_t a = (uint32_t)(uintptr_t)(SkLds*)lds;
+  asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base), "{m0}"(a) : "memory");
+}
+__device__ __forceinline__ void sk_dma4s(const void* base, uint32_t off, const void* lds) {
+  const uint32_t a = (uint32_t)(uintptr_t)(SkLds*)lds;
+  asm volatile("s_nop 0\n\tglobal_load_lds_dword %0, %1" ::"v"(off), "s"(base), "{m0}"(a) : "memory");
+}
+
 // Per-lane sources of a workgroup's loads, computed once; group g adds g times a stride.
 //   act  JS 1: this wave's block (4g + wave) of the 16-token tile, 2 KB, two instructions of 1 KB;
 //        JS 4: chain `wave` of the group's 4 blocks (512 bytes each), two blocks per instruction
@@ -81,11 +91,10 @@ __device__ __forceinline__ void sk_dma4(const void* src, const void* lds) {
 //   qs   JS 4: row lane (0..15) of the workgroup, chain `wave`; JS 1: row lane (0..63), chain `wave`
 //   sc   the 8 bytes of the group's 4 fp16 scales of one row, as two dwords (JS 4: lanes 0..31 take
 //        the 16 rows; JS 1: lanes 0..31 take rows 16 wave .. 16 wave + 15)
-// Blocks past nb and groups past ng are clamped to the last ones.
+// Blocks past nb and groups past ng are clamped to the last ones (JS 4: SkCursor stops at the last group).
 template <int JS>
 struct SkSrc {
-  const uint4* act;      // JS 1: block `wave` of group 0 of the tile; JS 4: the lane's uint4 of chain `wave` of block 0
-  const float* dx;       // JS 4: the lane's token scale in block 0
+  const uint4* act;      // JS 1: block `wave` of group 0 of the tile
   const uint4* qs;       // group 0
   const uint32_t* sc;    // group 0 (dword 0 of the row's 4-scale half of a uint4)
   int nb, ng, wave, lane;
@@ -101,29 +110,60 @@ struct SkSrc {
     const int gpr = hd >> 4, head = rg / gpr, p = rg - head * gpr;
     return head * hd + (l < 8 ? 8 * p + l : (hd >> 1) + 8 * p + l - 8);
   }
-  __device__ __forceinline__ SkSrc(const Q4Mat& W, const uint4* xt, int xstride, int T, int R0, int ffn = 0,
-                                   int hd = 0) {
+  __device__ __forceinline__ SkSrc(const Q4Mat& W, const uint4* xt, int xstride, int T, int R0, int ffn = 0) {
     lane = threadIdx.x & 63;
     wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     nb = W.nb;
     ng = W.ng;
     act = xt + (size_t)T * xstride * kXhBlock;
-    dx = reinterpret_cast<const float*>(act + 128) + (lane & 15);
-    const int tile = R0 >> 6, rr0 = R0 & 63;
-    if (JS == 4) act += wave * 32 + (lane & 31);
-    if (JS == 4 && hd > 0) {
-      const int rq = rope_row(R0 >> 4, hd, lane & 15), rs = rope_row(R0 >> 4, hd, (lane >> 1) & 15);
-      qs = W.qs + ((size_t)(rq >> 6) * ng * 64 + (rq & 63)) * 4 + wave;
-      sc = reinterpret_cast<const uint32_t*>(W.d + (size_t)(rs >> 6) * W.nb8 * 64 + (rs & 63)) + (lane & 1);
-    } else if (JS == 4) {
-      qs = W.qs + ((size_t)tile * ng * 64 + rr0 + (lane & 15)) * 4 + wave;
-      sc = reinterpret_cast<const uint32_t*>(W.d + (size_t)tile * W.nb8 * 64 + rr0 + ((lane >> 1) & 15)) +
-           (lane & 1);
-    } else {
-      const int rq = row_of(R0, ffn, lane), rs = row_of(R0, ffn, 16 * wave + ((lane >> 1) & 15));
-      qs = W.qs + ((size_t)(rq >> 6) * ng * 64 + (rq & 63)) * 4 + wave;
-      sc = reinterpret_cast<const uint32_t*>(W.d + (size_t)(rs >> 6) * W.nb8 * 64 + (rs & 63)) + (lane & 1);
-    }
+    const int rq = row_of(R0, ffn, lane), rs = row_of(R0, ffn, 16 * wave + ((lane >> 1) & 15));
+    qs = W.qs + ((size_t)(rq >> 6) * ng * 64 + (rq & 63)) * 4 + wave;
+    sc = reinterpret_cast<const uint32_t*>(W.d + (size_t)(rs >> 6) * W.nb8 * 64 + (rs & 63)) + (lane & 1);
+  }
+};
+
+// JS 4's loads: wave-uniform bases and byte offsets per lane that advance by a group's stride with each
+// issue (and stay at the last group, which the issues past it repeat), so a group's five addresses are
+// five additions.  Formed anew from the group number they were 64-bit products and clamps, a third of a
+// group's instructions in a kernel that one wave per SIMD runs (23 tokens through the 0.5B shape 1,432 ->
+// 1,396 us, 4 steps of 32 sequences of the 1.5B shape 12.82 -> 12.56 ms).
+struct SkCursor {
+  const void *abase, *qbase, *sbase;
+  uint32_t a, d, q, s;
+  int g, ng;
+  static constexpr uint32_t BLOCK = kXhBlock * 16;
+  // row group of rows R0 .. R0 + 15, or with hd > 0 of RoPE pairs (SkSrc::rope_row)
+  __device__ __forceinline__ SkCursor(const Q4Mat& W, const uint4* xt, int xstride, int T, int R0, int hd) {
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int rq = hd > 0 ? SkSrc<4>::rope_row(R0 >> 4, hd, lane & 15) : R0 + (lane & 15);
+    const int rs = hd > 0 ? SkSrc<4>::rope_row(R0 >> 4, hd, (lane >> 1) & 15) : R0 + ((lane >> 1) & 15);
+    const int t0 = (hd > 0 ? (R0 >> 4) / (hd >> 4) * hd : R0) >> 6;         // tile of the first row
+    abase = xt + (size_t)T * xstride * kXhBlock;
+    qbase = W.qs + (size_t)t0 * W.ng * 256;
+    sbase = W.d + (size_t)t0 * W.nb8 * 64;
+    a = (lane >> 5) * BLOCK + (wave * 32 + (lane & 31)) * 16;               // block lane / 32 of the group
+    d = (lane >> 4) * BLOCK + 2048 + (lane & 15) * 4;                       // block lane / 16
+    q = ((((rq >> 6) - t0) * W.ng * 64 + (rq & 63)) * 4 + wave) * 16;
+    s = (((rs >> 6) - t0) * W.nb8 * 64 + (rs & 63)) * 16 + (lane & 1) * 4;
+    g = 0;
+    ng = W.ng;
+  }
+  // the next group into this wave's part of a slot: five instructions
+  __device__ __forceinline__ void issue(unsigned char* w) {
+    using S = SkSlot<4>;
+    const int lane = threadIdx.x & 63;
+    sk_dma16s(abase, a, w);
+    sk_dma16s(abase, a + 2 * BLOCK, w + 1024);
+    sk_dma4s(abase, d, w + S::oDX);
+    if (lane < 16) sk_dma16s(qbase, q, w + S::oQS);
+    if (lane < 32) sk_dma4s(sbase, s, w + S::oSC);
+    const bool more = g + 1 < ng;
+    const uint32_t step = more ? 4 * BLOCK : 0;
+    a += step;
+    d += step;
+    q += more ? 4096 : 0;
+    s += more ? ((g & 1) ? 1016 : 8) : 0;                                   // 4 scales on, or the next 8 scales' uint4
+    g += more ? 1 : 0;
   }
 };
 
@@ -134,20 +174,6 @@ __device__ __forceinline__ void sk_issue(const unsigned char* slot, const SkSrc<
   const int lane = src.lane, wave = src.wave;
   g = g < src.ng ? g : src.ng - 1;
   const uint32_t* scg = src.sc + (size_t)(g >> 1) * 256 + ((g & 1) << 1);   // 64 rows x 4 dwords per uint4 group
-  if (JS == 4) {
-    // this wave's part of the slot: blocks 4g .. 4g + 3 of chain `wave` (lanes 0..31 and 32..63
-    // take one block each per instruction), the 4 blocks' dx, the rows' words and scales
-    unsigned char* const w = const_cast<unsigned char*>(slot) + wave * S::WAVE;
-    const int last = src.nb - 1;
-    const int b0 = min(4 * g + (lane >> 5), last), b1 = min(4 * g + 2 + (lane >> 5), last);
-    const int bd = min(4 * g + (lane >> 4), last);
-    sk_dma16(src.act + (size_t)b0 * kXhBlock, w);
-    sk_dma16(src.act + (size_t)b1 * kXhBlock, w + 1024);
-    sk_dma4(src.dx + (size_t)bd * kXhBlock * 4, w + S::oDX);
-    if (lane < 16) sk_dma16(src.qs + (size_t)g * 256, w + S::oQS);
-    if (lane < 32) sk_dma4(scg, w + S::oSC);
-    return;
-  }
   int b = 4 * g + wave;
   b = b < src.nb ? b : src.nb - 1;
   const uint4* a = src.act + (size_t)b * kXhBlock;
@@ -283,7 +309,8 @@ __global__ __launch_bounds__(256) void k_gemm_sk(Q4Mat W, const uint4* __restric
   __shared__ __align__(16) unsigned char q0[S::BYTES], q1[S::BYTES], q2[S::BYTES], q3[S::BYTES], q4[S::BYTES],
       q5[S::BYTES], q6[S::BYTES], q7[S::BYTES];
   unsigned char* const ring[8] = {q0, q1, q2, q3, q4, q5, q6, q7};
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, li = lane & 15, kg = lane >> 4;
+  const int tid = threadIdx.x, lane = tid & 63, li = lane & 15, kg = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   // nrg row groups (16 rows for JS 4, 64 for JS 1, one 32-value block of gate and up for EPI 1)
   // times ceil(M / 16) token tiles, placed by sk_place
   const int nrg = EPI == 1 ? ffn / 32 : JS == 4 ? W.Np / 16 : W.Np / 64;
@@ -292,7 +319,8 @@ __global__ __launch_bounds__(256) void k_gemm_sk(Q4Mat W, const uint4* __restric
   const int R0 = EPI == 1 ? rgi * 32 : JS == 4 ? rgi * 16 : rgi * 64;
   const int ng = W.ng;
   const SkB bop(kg);
-  const SkSrc<JS> src(W, xt, xstride, T, R0, EPI == 1 ? ffn : 0, EPI == 2 ? rp.hd : 0);
+  const SkSrc<JS> src(W, xt, xstride, T, R0, EPI == 1 ? ffn : 0);                        // JS 1
+  SkCursor cur(W, xt, xstride, T, R0, EPI == 2 ? rp.hd : 0);                             // JS 4
   constexpr int NJ = JS == 4 ? 1 : 4;
   const int wrow = JS == 4 ? li : 16 * wave + li;            // this lane's weight row in the workgroup
   float acc[NJ][4];
@@ -359,7 +387,10 @@ __global__ __launch_bounds__(256) void k_gemm_sk(Q4Mat W, const uint4* __restric
   };
 
 #pragma unroll
-  for (int p = 0; p < R - 1; p++) sk_issue<JS>(ring[p], src, p);
+  for (int p = 0; p < R - 1; p++) {
+    if (JS == 4) cur.issue(ring[p] + wave * S::BYTES / 4);
+    else sk_issue<JS>(ring[p], src, p);
+  }
   if (JS == 4) {
     // Software pipeline over groups (JS 4; the 64-row layout has no registers to spare for it):
     // once group g's slot is free (its reads done), a wave reads group g + 1's operands from
@@ -369,7 +400,7 @@ __global__ __launch_bounds__(256) void k_gemm_sk(Q4Mat W, const uint4* __restric
     static_assert(R % 2 == 0, "register sets alternate with the group parity");
     Regs G[2];
     sk_wait<5 * (R - 2)>();                                  // group 0 has landed
-    sk_issue<JS>(ring[R - 1], src, R - 1);
+    cur.issue(ring[R - 1] + wave * S::WAVE);
     read(ring[0], G[0]);
     for (int g0 = 0; g0 < ng; g0 += R) {
 #pragma unroll
@@ -382,7 +413,7 @@ __global__ __launch_bounds__(256) void k_gemm_sk(Q4Mat W, const uint4* __restric
           // the same wait in a form the compiler's wait tracking sees: the registers read in the
           // previous step are ready, so computing from them does not wait for the reads below
           __builtin_amdgcn_s_waitcnt(0xC07F);                // lgkmcnt(0)
-          sk_issue<JS>(ring[u], src, g + R);
+          cur.issue(ring[u] + wave * S::WAVE);
           read(ring[(u + 1) % R], G[(u + 1) & 1]);
           compute(G[u & 1], g);
         }
