@@ -213,12 +213,13 @@ void q4hip_mv_destroy(q4hip_mv* m);
 /* The matvec of q4hip_mv_run with nothing allocated: no counterpart in the reference.  It is for
  * callers that cannot allocate device memory (code under HIP graph capture, serving loops and
  * harnesses that forbid hipMalloc).  x (K floats) and y (N floats) are device memory of the
- * handle's device, checked before anything is launched.  The int8 activation blocks go to a
- * library-owned static device buffer of Q4HIP_NOALLOC_MAX_K / 32 blocks (128 KB per device, held
- * until the process ends); K above Q4HIP_NOALLOC_MAX_K is rejected.  `stream` (a hipStream_t)
+ * handle's device, checked before anything is launched.  Rows of up to 480 blocks (K = 15360) are
+ * quantized by the projection itself; for wider ones, and where y overlaps x, the int8 activation
+ * blocks go to a library-owned static device buffer of Q4HIP_NOALLOC_MAX_K / 32 blocks (128 KB per
+ * device, held until the process ends); K above Q4HIP_NOALLOC_MAX_K is rejected.  `stream` (a hipStream_t)
  * NULL: the handle's stream, and the call waits for the result; otherwise the work is enqueued
- * on that stream and the call returns at once.  Every call on one device shares the buffer:
- * calls that overlap on one GPU (other streams, other threads, other handles) race. */
+ * on that stream and the call returns at once.  Calls that use the buffer share it per device: those
+ * that overlap on one GPU (other streams, other threads, other handles) race. */
 #define Q4HIP_NOALLOC_MAX_K 65536
 int q4hip_mv_run_noalloc(q4hip_mv* m, const float* x, float* y, void* stream);
 
