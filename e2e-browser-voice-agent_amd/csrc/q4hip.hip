@@ -24,6 +24,7 @@
 #include "kernels.h"
 #include "persistent.h"
 #include "q4hip.h"
+#include "route.h"
 
 using namespace q4;
 
@@ -135,9 +136,10 @@ __global__ __launch_bounds__(256) void k_quant(const float* __restrict__ in, int
 enum { OP_STORE = 0, OP_BIAS = 1, OP_ADD = 2 };   // put() of kernels.c:190-194
 
 // The nb activation blocks of one token into shared memory: copied, or (an fp32 activation) quantized
-// as k_quant<QM_PLAIN> does.  Every workgroup of a one-token projection quantizes the whole vector
-// for itself while its first weights load: 896 values are one work item for half the threads, less
-// than the launch of its own that it replaces (a call of the 896 x 896 matvec 6.8 -> 4.5 us).
+// as k_quant<QM_PLAIN> does.  Then every workgroup quantizes the whole vector for itself
+// (k_matvec_stream while its first weights load, the others before): 896 values are one work item for
+// half the threads, less than the launch of its own that it replaces (a call of the 896 x 896 matvec
+// 6.8 -> 4.5 us).  mv_quantizes_itself says for which matrices.
 __device__ __forceinline__ void stage_blocks(const uint4* __restrict__ xq, int nb, uint4* xs, int tid, int nthreads) {
   for (int i = tid; i < nb * 4; i += nthreads) xs[i] = xq[i];
 }
@@ -450,10 +452,8 @@ __global__ __launch_bounds__(kSplitThreads) void k_matvec_split(Q4Mat W, const X
   }
 }
 
-// Blocks per row from which one-token projections use k_matvec_split.
-constexpr int kSplitMinBlocks = 64;
-// The widest row it takes: activation blocks and terms in shared memory.
-constexpr int kSplitMaxBlocks = 480;
+// One-token projections of kSplitMinBlocks .. kSplitMaxBlocks blocks a row use k_matvec_split; the widest
+// is bound by its activation blocks and terms in shared memory.
 inline size_t split_lds(int nb) { return (size_t)nb * 320; }
 
 // The widest row of a one-token projection on k_matvec (rows wider than k_matvec_split takes):
@@ -3810,9 +3810,9 @@ int q4hip_mv_run_noalloc(q4hip_mv* m, const float* x, float* y, void* stream) {
   if (K > Q4HIP_NOALLOC_MAX_K)
     return fail(Q4HIP_EINVAL, "K = %d exceeds the no-allocation limit of %d", K, Q4HIP_NOALLOC_MAX_K);
   HIPCHK(hipSetDevice(m->device));
-  // x is quantized once, in a launch of its own, for rows past kSplitMaxBlocks and where y overlaps it
-  // (a workgroup's results would change what a later one reads)
-  const bool fused = m->W.nb <= kSplitMaxBlocks && (y >= x + K || x >= y + N);
+  // where y overlaps x, too, x is quantized in a launch of its own (a workgroup's results would change
+  // what a later one reads)
+  const bool fused = mv_quantizes_itself(N, m->W.nb) && (y >= x + K || x >= y + N);
   uint4* xq = nullptr;
   int rc = fused ? Q4HIP_OK : scratch_on(m->device, &xq);
   if (rc == Q4HIP_OK) rc = check_device_span(x, (size_t)K * 4, m->device, "x");

@@ -213,10 +213,11 @@ void q4hip_mv_destroy(q4hip_mv* m);
 /* The matvec of q4hip_mv_run with nothing allocated: no counterpart in the reference.  It is for
  * callers that cannot allocate device memory (code under HIP graph capture, serving loops and
  * harnesses that forbid hipMalloc).  x (K floats) and y (N floats) are device memory of the
- * handle's device, checked before anything is launched.  Rows of up to 480 blocks (K = 15360) are
- * quantized by the projection itself; for wider ones, and where y overlaps x, the int8 activation
- * blocks go to a library-owned static device buffer of Q4HIP_NOALLOC_MAX_K / 32 blocks (128 KB per
- * device, held until the process ends); K above Q4HIP_NOALLOC_MAX_K is rejected.  `stream` (a hipStream_t)
+ * handle's device, checked before anything is launched.  The projection quantizes x itself for rows of
+ * up to 63 blocks and, with N moderate (28672 rows at K = 2048, 14656 at K = 15360), of up to 480.  For
+ * other matrices, and where y overlaps x, the int8 activation blocks go to a library-owned static device
+ * buffer of Q4HIP_NOALLOC_MAX_K / 32 blocks (128 KB per device, held until the process ends); K above
+ * Q4HIP_NOALLOC_MAX_K is rejected.  `stream` (a hipStream_t)
  * NULL: the handle's stream, and the call waits for the result; otherwise the work is enqueued
  * on that stream and the call returns at once.  Calls that use the buffer share it per device: those
  * that overlap on one GPU (other streams, other threads, other handles) race. */
