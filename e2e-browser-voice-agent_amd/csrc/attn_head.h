@@ -25,22 +25,14 @@
 
 #include "gemm_sk.h"
 #include "kernels.h"
+#include "route.h"
 
 namespace q4 {
 
 constexpr int kHeadThreads = 256;
 constexpr int kHeadStage = 8192;        // bytes of a K stage: 64 rows x 128 bytes
 constexpr int kHeadMaxLds = 160 * 1024;
-
-// Floats of the row of scores (exponentials, probabilities): every position, the +0 past them for
-// ordered_sum_wave and the rest of the last P.V chunk.
-__host__ __device__ inline int head_row(int ctx) { return ((ctx + 31) & ~31) + 128 + (ctx >> 6); }
-// Bytes shared by the K stages (two per wave; three were no faster) and the V slots.
-constexpr int kHeadStageBytes = kHeadThreads / 64 * 2 * kHeadStage;
-template <int HD>
-inline size_t attn_head_lds(int ctx) {
-  return (size_t)kHeadStageBytes + (size_t)(head_row(ctx) + 16 + kHeadThreads / 64 * HD) * sizeof(float);
-}
+static_assert(kHeadStageBytes == kHeadThreads / 64 * 2 * kHeadStage, "two K stages per wave (three were no faster)");
 // Workgroups: units (row, kv head) dealt to the 8 XCDs, the G heads of a unit 8 workgroups apart.
 inline unsigned attn_head_grid(int rows, int KVH, int G) {
   return (unsigned)((rows * KVH + kXcds - 1) / kXcds * kXcds * G);
@@ -296,7 +288,8 @@ struct HeadPv<128, KT> {
 template <int HD, class KT>
 __global__ __launch_bounds__(kHeadThreads, 2) void k_attn_head(const float* __restrict__ qkv, int QKV, int H, int KVH,
                                                                const KT* __restrict__ kc, const KT* __restrict__ vc,
-                                                               int ctx, int layer, const int* __restrict__ pos, int B,
+                                                               int ctx, int end, int layer,
+                                                               const int* __restrict__ pos, int B,
                                                                size_t seq_stride, uint4* __restrict__ xq, int xstride,
                                                                uint4* __restrict__ xh) {
   constexpr int NW = kHeadThreads / 64, RB = HD * (int)sizeof(KT), NP = RB / 128;   // bytes, 128-byte pieces of a row
@@ -310,7 +303,7 @@ __global__ __launch_bounds__(kHeadThreads, 2) void k_attn_head(const float* __re
   const int T = pos[b] + 1;
   unsigned char* const stage = reinterpret_cast<unsigned char*>(lsm);
   float* const e = lsm + kHeadStageBytes / 4;      // scores, then exponentials, then probabilities
-  float* const red = e + head_row(ctx);
+  float* const red = e + head_row(end);
   const size_t cb = (size_t)b * seq_stride + ((size_t)layer * KVH + g) * ctx * HD;
 
   // ---- scores: wave w takes positions 64 c .. 64 c + 63 of the chunks c = w mod 4

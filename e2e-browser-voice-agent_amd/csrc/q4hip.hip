@@ -2463,9 +2463,10 @@ size_t attn_pv_lds(int H, int KVH, int ctx) {
 }
 
 // With xq, the P.V kernel also writes the quantized activation of att (k_quant<QM_PLAIN>'s output).
+// end: one past the last position of any row (a captured step, whose position moves: ctx).
 template <class KT>
 void launch_attn_list_t(hipStream_t s, int HD, int B, int H, int KVH, const float* qkv, int QKV, const KT* kc,
-                        const KT* vc, int ctx, int layer, float* sc, float* att, int D, const int* pos,
+                        const KT* vc, int ctx, int end, int layer, float* sc, float* att, int D, const int* pos,
                         size_t seq_stride, uint4* xq, int xstride, uint4* xh) {
   const dim3 sg((unsigned)((ctx + kScoreRows - 1) / kScoreRows), (unsigned)KVH, (unsigned)B);
   const unsigned units = (unsigned)KVH * (unsigned)B, pg = units * (unsigned)(HD / kPvCols);
@@ -2474,15 +2475,16 @@ void launch_attn_list_t(hipStream_t s, int HD, int B, int H, int KVH, const floa
   const int Gq = H / KVH;
   int dev = 0;
   if (xq && !pv_tiles_off() && (seq_stride != 0 || B == 1 || (!attn_rows_off() && B * H <= head_max_units(HD))) &&
-      (HD == 64 ? attn_head_lds<64>(ctx) : attn_head_lds<128>(ctx)) <= (size_t)kHeadMaxLds &&
+      attn_head_lds(HD, end) <= (size_t)kHeadMaxLds &&
       hipGetDevice(&dev) == hipSuccess && attn_head_setup(dev)) {
     const unsigned hg = attn_head_grid(B, KVH, Gq);
+    const size_t hlds = attn_head_lds(HD, end);
     if (HD == 64)
-      k_attn_head<64, KT><<<hg, kHeadThreads, attn_head_lds<64>(ctx), s>>>(qkv, QKV, H, KVH, kc, vc, ctx, layer, pos, B,
-                                                                           seq_stride, xq, xstride, xh);
+      k_attn_head<64, KT><<<hg, kHeadThreads, hlds, s>>>(qkv, QKV, H, KVH, kc, vc, ctx, end, layer, pos, B, seq_stride, xq,
+                                                         xstride, xh);
     else
-      k_attn_head<128, KT><<<hg, kHeadThreads, attn_head_lds<128>(ctx), s>>>(qkv, QKV, H, KVH, kc, vc, ctx, layer, pos, B,
-                                                                             seq_stride, xq, xstride, xh);
+      k_attn_head<128, KT><<<hg, kHeadThreads, hlds, s>>>(qkv, QKV, H, KVH, kc, vc, ctx, end, layer, pos, B, seq_stride, xq,
+                                                          xstride, xh);
     return;
   }
   if (seq_stride == 0 && B > 1 && !pv_tiles_off() && !attn_rows_off() && HD == 64 && Gq <= kMaxGroup &&
@@ -2530,13 +2532,13 @@ void launch_attn_list_t(hipStream_t s, int HD, int B, int H, int KVH, const floa
 
 // kc, vc: fp32 caches, or fp16 ones when kv16.
 void launch_attn_list(hipStream_t s, int HD, int B, int H, int KVH, const float* qkv, int QKV, const void* kc,
-                      const void* vc, bool kv16, int ctx, int layer, float* sc, float* att, int D, const int* pos,
+                      const void* vc, bool kv16, int ctx, int end, int layer, float* sc, float* att, int D, const int* pos,
                       size_t seq_stride, uint4* xq = nullptr, int xstride = 0, uint4* xh = nullptr) {
   if (kv16)
-    launch_attn_list_t<kvhalf>(s, HD, B, H, KVH, qkv, QKV, (const kvhalf*)kc, (const kvhalf*)vc, ctx, layer, sc, att,
+    launch_attn_list_t<kvhalf>(s, HD, B, H, KVH, qkv, QKV, (const kvhalf*)kc, (const kvhalf*)vc, ctx, end, layer, sc, att,
                                D, pos, seq_stride, xq, xstride, xh);
   else
-    launch_attn_list_t<float>(s, HD, B, H, KVH, qkv, QKV, (const float*)kc, (const float*)vc, ctx, layer, sc, att, D,
+    launch_attn_list_t<float>(s, HD, B, H, KVH, qkv, QKV, (const float*)kc, (const float*)vc, ctx, end, layer, sc, att, D,
                               pos, seq_stride, xq, xstride, xh);
 }
 
@@ -2565,8 +2567,9 @@ bool attn_list_ok(int H, int KVH, int HD, int ctx) {
   return true;
 }
 
-// One pass over M <= MT tokens at device position st->pos0 (forward_pass, kernels.c:306-415).
-void enqueue_pass(q4hip* h, int M, bool want_logits) {
+// One pass over M <= MT tokens at device position st->pos0 (forward_pass, kernels.c:306-415), which ends
+// at position `end` at most.
+void enqueue_pass(q4hip* h, int M, bool want_logits, int end) {
   const int D = h->D, F = h->F, HD = h->HD, QKV = h->QKV;
   hipStream_t s = h->stream;
   uint4* xh = M > 1 ? h->xh : nullptr;
@@ -2598,7 +2601,7 @@ void enqueue_pass(q4hip* h, int M, bool want_logits) {
     prof_mark(h, Q4HIP_PROF_ATTN);
     bool quantized = false;                 // the list P.V kernel wrote xq (and xh) itself
     if (M > 1 && h->ascr && h->list_attn == 1) {
-      launch_attn_list(s, HD, M, h->H, h->KVH, h->qkv, QKV, h->kc, h->vc, h->kv16, h->ctx, l, h->ascr, h->att, D, h->tpos, 0,
+      launch_attn_list(s, HD, M, h->H, h->KVH, h->qkv, QKV, h->kc, h->vc, h->kv16, h->ctx, end, l, h->ascr, h->att, D, h->tpos, 0,
                        h->xq, h->xstride, xh);
       quantized = true;
     } else if (M > 1 && h->ascr) {
@@ -2616,7 +2619,7 @@ void enqueue_pass(q4hip* h, int M, bool want_logits) {
         k_attn_prefill<128, float><<<ag, 256, 0, s>>>(h->qkv, QKV, h->H, h->KVH, (const float*)h->kc, (const float*)h->vc, h->ctx, l,
                                                       h->att, D, h->st, M, h->ascr);
     } else if (M == 1 && h->ascr && h->list_attn == 1) {
-      launch_attn_list(s, HD, 1, h->H, h->KVH, h->qkv, QKV, h->kc, h->vc, h->kv16, h->ctx, l, h->ascr, h->att, D, &h->st->pos0, 0,
+      launch_attn_list(s, HD, 1, h->H, h->KVH, h->qkv, QKV, h->kc, h->vc, h->kv16, h->ctx, end, l, h->ascr, h->att, D, &h->st->pos0, 0,
                        h->xq, h->xstride, xh);
       quantized = true;
     } else if (HD == 64 && h->kv16) {
@@ -2925,7 +2928,7 @@ int build_graph(q4hip* h) {
     (void)hipGetLastError();
     return Q4HIP_OK;
   }
-  enqueue_pass(h, 1, true);
+  enqueue_pass(h, 1, true, h->ctx);
   hipError_t e = hipStreamEndCapture(h->stream, &g);
   if (e == hipSuccess) e = hipGraphInstantiate(&h->graph, g, nullptr, nullptr, 0);
   if (g) (void)hipGraphDestroy(g);
@@ -2939,7 +2942,7 @@ int build_graph(q4hip* h) {
 
 void decode_step(q4hip* h) {
   if (h->graph) (void)hipGraphLaunch(h->graph, h->stream);
-  else enqueue_pass(h, 1, true);
+  else enqueue_pass(h, 1, true, h->ctx);
 }
 
 }  // namespace
@@ -3162,7 +3165,7 @@ int q4hip_forward(q4hip* h, const int* ids, int n, int pos, int* next) {
       HIPCHK(hipGraphLaunch(h->graph, h->stream));
       h->last_mode = Q4HIP_DECODE_GRAPH;
     } else {
-      enqueue_pass(h, k, last);
+      enqueue_pass(h, k, last, pos + c + k);
       if (k == 1) h->last_mode = Q4HIP_DECODE_GRAPH;
     }
   }
@@ -3303,7 +3306,7 @@ int q4hip_profile_pass(q4hip* h, const int* ids, int ntok, int pos, float* us, i
   k_set_pos<<<1, 64, 0, h->stream>>>(h->st, pos);
   std::vector<std::pair<int, hipEvent_t>> marks;
   h->prof = &marks;
-  enqueue_pass(h, ntok, true);
+  enqueue_pass(h, ntok, true, pos + ntok);
   h->prof = nullptr;
   hipError_t e = hipStreamSynchronize(h->stream);
   for (int i = 0; i < Q4HIP_PROF_N; i++) us[i] = 0.0f;
@@ -3399,8 +3402,8 @@ struct q4hip_batch {
 namespace {
 
 // One decode step of all B sequences: tokens bt->tok at positions bt->pos; the greedy tokens go to
-// bt->tok (and out[0..B) when given) and every position advances by one.
-void enqueue_batch_step(q4hip_batch* bt, int* out) {
+// bt->tok (and out[0..B) when given) and every position advances by one, to `end` at most.
+void enqueue_batch_step(q4hip_batch* bt, int* out, int end) {
   q4hip* h = bt->h;
   const int B = bt->B, D = h->D, F = h->F, HD = h->HD, QKV = h->QKV;
   hipStream_t s = h->stream;
@@ -3423,7 +3426,7 @@ void enqueue_batch_step(q4hip_batch* bt, int* out) {
                                                                         (float*)bt->kc, (float*)bt->vc, h->ctx, l,
                                                                         bt->pos, bt->seq_stride);
     }
-    launch_attn_list(s, HD, B, h->H, h->KVH, h->qkv, QKV, bt->kc, bt->vc, h->kv16, h->ctx, l, bt->sc, h->att, D, bt->pos,
+    launch_attn_list(s, HD, B, h->H, h->KVH, h->qkv, QKV, bt->kc, bt->vc, h->kv16, h->ctx, end, l, bt->sc, h->att, D, bt->pos,
                      bt->seq_stride, h->xq, h->xstride, xh);
     launch_matvec<OP_ADD>(s, y.o, h->xq, h->xstride, B, h->x, D, nullptr, xh);
     launch_quant<QM_NORM>(s, B, h->x, D, D, y.ffn_norm, h->eps, h->xq, h->xstride, 0, xh);
@@ -3545,7 +3548,7 @@ int q4hip_batch_prefill(q4hip_batch* bt, int seq, const int* ids, int n, int pos
   for (int c = 0; e == hipSuccess && c < n; c += h->MT) {
     const int k = std::min(h->MT, n - c);
     k_set_pos<<<1, 64, 0, h->stream>>>(h->st, pos + c);
-    enqueue_pass(h, k, c + k >= n);
+    enqueue_pass(h, k, c + k >= n, pos + c + k);
   }
   h->kc = kc;
   h->vc = vc;
@@ -3586,7 +3589,8 @@ static int run_batch(q4hip_batch* bt, const int* first, const int* pos, int step
     HIPCHK(hipEventCreate(&e1));
     HIPCHK(hipEventRecord(e0, h->stream));
   }
-  for (int i = 0; i < steps; i++) enqueue_batch_step(bt, bt->out + (size_t)i * B);
+  const int end = *std::max_element(pos, pos + B) + steps;
+  for (int i = 0; i < steps; i++) enqueue_batch_step(bt, bt->out + (size_t)i * B, end);
   if (ms) HIPCHK(hipEventRecord(e1, h->stream));
   HIPCHK(hipGetLastError());
   HIPCHK(hipStreamSynchronize(h->stream));

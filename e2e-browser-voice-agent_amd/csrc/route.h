@@ -29,4 +29,17 @@ inline bool mv_quantizes_itself(int N, int nb) {
   return wgs <= 1792 && wgs * nb <= 440000;
 }
 
+// ---- attention
+
+// Shared memory of k_attn_head, whose workgroup takes one row and head: the K stages and V slots, the row
+// of scores (exponentials, probabilities) of up to `end` positions -- every position, the +0 past them
+// for ordered_sum_wave and the rest of the last P.V chunk -- and the waves' q and reductions.  `end` is
+// one past the last position that any row of the call looks at, not the context's size: two workgroups
+// fit a CU up to about 3,600 positions (head_dim 64; 3,300 with 128), one beyond.
+constexpr int kHeadStageBytes = 64 * 1024;
+constexpr int head_row(int end) { return ((end + 31) & ~31) + 128 + (end >> 6); }
+constexpr size_t attn_head_lds(int HD, int end) {
+  return (size_t)kHeadStageBytes + (size_t)(head_row(end) + 16 + 4 * HD) * sizeof(float);
+}
+
 }  // namespace q4

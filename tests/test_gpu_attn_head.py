@@ -1,7 +1,7 @@
 """The one-(row, head)-per-workgroup attention against the oracle: contexts at the edges of its 64-position
 K chunks and of the 64- and 128-position chunks of P.V, in a batch of sequences, a short pass at a
 position, and one-token steps past the length from which the softmax sum is formed by the whole wave.
-Tokens equal, logits bit for bit.
+Tokens equal, logits bit for bit.  Its time follows the positions in use, not the size of the context.
 """
 import numpy as np
 import pytest
@@ -75,3 +75,25 @@ def test_sum_by_the_wave(name, kv):
     finally:
         g.close()
         o.close()
+
+
+def test_time_follows_the_positions_not_the_context():
+    """36 rows of 14 heads are 504 workgroups: two fit a CU with the shared memory of 36 positions, one with
+    that of a 4,400-position context (attention 1.5 times as long).  Best of 9 in turn; 1.25 is half way."""
+    import q4hip
+    shape = synth.Shape(896, 8, 256, 14, 2, 512)
+    t = synth.make_model(shape, 96)
+    ids = synth.prompt_ids(5, 36, shape.vocab)
+    models = [q4hip.Model(shape, ctx=ctx) for ctx in (512, 4400)]
+    best = [1e9, 1e9]
+    try:
+        for m in models:
+            m.load(t)
+        for _ in range(9):
+            for i, m in enumerate(models):
+                best[i] = min(best[i], m.profile_pass(ids, 0)["attention"])
+    finally:
+        for m in models:
+            m.close()
+    print(f"attention of 8 layers: {best[0]:.1f} us in 512 positions, {best[1]:.1f} in 4,400", flush=True)
+    assert best[1] < 1.25 * best[0]
