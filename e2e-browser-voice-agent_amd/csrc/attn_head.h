@@ -33,10 +33,6 @@ constexpr int kHeadThreads = 256;
 constexpr int kHeadStage = 8192;        // bytes of a K stage: 64 rows x 128 bytes
 constexpr int kHeadMaxLds = 160 * 1024;
 static_assert(kHeadStageBytes == kHeadThreads / 64 * 2 * kHeadStage, "two K stages per wave (three were no faster)");
-// Workgroups: units (row, kv head) dealt to the 8 XCDs, the G heads of a unit 8 workgroups apart.
-inline unsigned attn_head_grid(int rows, int KVH, int G) {
-  return (unsigned)((rows * KVH + kXcds - 1) / kXcds * kXcds * G);
-}
 
 // Four neighbouring cache values, and a product with one: rounded once to fp32.  An fp16 value is
 // widened inside the instruction (v_fma_mix with an addend of +0, which can only turn a product of

@@ -25,6 +25,7 @@
 // (valid memory, never used).
 #pragma once
 #include "kernels.h"
+#include "route.h"
 
 namespace q4 {
 
@@ -217,7 +218,6 @@ struct SkB {
 // and the XCD's L2 serves the second reader, where row-group-fastest order with a row-group count
 // that is not a multiple of 8 (the output head: 2374 groups of 64 rows) put them on different XCDs
 // a whole pass apart.  Returns false for padding workgroups (row group past the last).
-constexpr int kXcds = 8;
 constexpr int kSkPairTiles = 4;
 
 __host__ __device__ inline bool sk_paired(int ntiles, bool by_tile) {

@@ -1725,7 +1725,7 @@ struct q4hip {
   State* st = nullptr;
   int* pin_ids = nullptr;     // pinned staging: token ids in, ids out
   int* pin_next = nullptr;
-  hipGraphExec_t graph = nullptr;
+  hipGraphExec_t graph[2] = {nullptr, nullptr};   // the captured one-token step, by its attention kernel (step_graph)
   bool graph_failed = false;
   int last_mode = 0;
   // persistent decode (one launch per forward/generate call)
@@ -2422,17 +2422,6 @@ void launch_quant(hipStream_t s, int rows, const float* in, int ld_in, int n, co
   k_quant<MODE><<<xh && rows >= 128 ? 8 * ((rows + 7) / 8) : rows, 256, lds, s>>>(in, ld_in, n, w, eps, xq, xstride, m_first, xh, rows);
 }
 
-// Largest prompt pass, in (row, head) units, that k_attn_head takes: from there on the kernels that
-// read a K row once for all heads of a group are faster.  head_dim 64, against k_attn_rows, whole
-// passes of the 0.5B shape (14 heads) at position 0 and at 600: 48 tokens 1.44 / 1.79 against 1.53 /
-// 1.87 ms, 72 tokens 1.65 / 2.08 against 1.75 / 2.06 ms, 96 tokens 1.88 / 2.49 against 1.88 / 2.19 ms.
-// head_dim 128, against three launches, 1.5B shape (12 heads): 48 tokens 2.74 against 3.08 ms, 224
-// tokens 6.85 against 6.93 ms, 600 tokens 15.3 against 13.9 ms.  Batches of sequences share no cache
-// rows between them and take it at any size (32 sequences of 1,026 positions, 1.5B shape: 29.6 us a
-// layer against 33.0 for k_attn_scores_list and k_attn_pv_list), as does a single token (700
-// positions: 15.5 against 27.2 us).
-inline int head_max_units(int HD) { return HD == 64 ? 1024 : 3072; }
-
 // Raise k_attn_head's shared-memory limit once per device, with that device current (before any
 // graph capture; attn_list_ok calls it).
 bool attn_head_setup(int device) {
@@ -2463,10 +2452,9 @@ size_t attn_pv_lds(int H, int KVH, int ctx) {
 }
 
 // With xq, the P.V kernel also writes the quantized activation of att (k_quant<QM_PLAIN>'s output).
-// end: one past the last position of any row (a captured step, whose position moves: ctx).
 template <class KT>
 void launch_attn_list_t(hipStream_t s, int HD, int B, int H, int KVH, const float* qkv, int QKV, const KT* kc,
-                        const KT* vc, int ctx, int end, int layer, float* sc, float* att, int D, const int* pos,
+                        const KT* vc, int ctx, AttnSpan sp, int layer, float* sc, float* att, int D, const int* pos,
                         size_t seq_stride, uint4* xq, int xstride, uint4* xh) {
   const dim3 sg((unsigned)((ctx + kScoreRows - 1) / kScoreRows), (unsigned)KVH, (unsigned)B);
   const unsigned units = (unsigned)KVH * (unsigned)B, pg = units * (unsigned)(HD / kPvCols);
@@ -2474,28 +2462,31 @@ void launch_attn_list_t(hipStream_t s, int HD, int B, int H, int KVH, const floa
   const size_t lds = attn_pv_lds(H, KVH, ctx);
   const int Gq = H / KVH;
   int dev = 0;
-  if (xq && !pv_tiles_off() && (seq_stride != 0 || B == 1 || (!attn_rows_off() && B * H <= head_max_units(HD))) &&
-      attn_head_lds(HD, end) <= (size_t)kHeadMaxLds &&
+  const bool pass = seq_stride == 0 && B > 1;                // a prompt pass: rows share one cache
+  if (xq && !pv_tiles_off() && !(pass && attn_rows_off()) &&
+      (pass ? head_takes_pass(B, H, KVH, HD, sizeof(KT) == 2, sp)
+            : head_takes_rows(B, H, KVH, HD, sizeof(KT) == 2, sp)) &&
+      attn_head_lds(HD, sp.end) <= (size_t)kHeadMaxLds &&
       hipGetDevice(&dev) == hipSuccess && attn_head_setup(dev)) {
     const unsigned hg = attn_head_grid(B, KVH, Gq);
-    const size_t hlds = attn_head_lds(HD, end);
+    const size_t hlds = attn_head_lds(HD, sp.end);
     if (HD == 64)
-      k_attn_head<64, KT><<<hg, kHeadThreads, hlds, s>>>(qkv, QKV, H, KVH, kc, vc, ctx, end, layer, pos, B, seq_stride, xq,
+      k_attn_head<64, KT><<<hg, kHeadThreads, hlds, s>>>(qkv, QKV, H, KVH, kc, vc, ctx, sp.end, layer, pos, B, seq_stride, xq,
                                                          xstride, xh);
     else
-      k_attn_head<128, KT><<<hg, kHeadThreads, hlds, s>>>(qkv, QKV, H, KVH, kc, vc, ctx, end, layer, pos, B, seq_stride, xq,
+      k_attn_head<128, KT><<<hg, kHeadThreads, hlds, s>>>(qkv, QKV, H, KVH, kc, vc, ctx, sp.end, layer, pos, B, seq_stride, xq,
                                                           xstride, xh);
     return;
   }
-  if (seq_stride == 0 && B > 1 && !pv_tiles_off() && !attn_rows_off() && HD == 64 && Gq <= kMaxGroup &&
+  if (pass && !pv_tiles_off() && !attn_rows_off() && HD == 64 && Gq <= kMaxGroup &&
       attn_rows_lds(Gq, ctx) <= (size_t)kAttnRowsMaxLds &&
       (attn_rows_lds(Gq, ctx) <= 64 * 1024 || (hipGetDevice(&dev) == hipSuccess && attn_rows_setup(dev)))) {
-    // a prompt pass in one launch: scores and probabilities stay in shared memory
+    // one launch: scores and probabilities stay in shared memory
     k_attn_rows<KT><<<dim3((unsigned)KVH, (unsigned)B), kAttnRowsThreads, attn_rows_lds(Gq, ctx), s>>>(
         qkv, QKV, H, KVH, kc, vc, ctx, layer, pos, B, att, D, xq, xstride, xh);
     return;
   }
-  if (seq_stride == 0 && B > 1 && !pv_tiles_off()) {   // a prompt pass: rows share one cache
+  if (pass && !pv_tiles_off()) {
     const dim3 tg((unsigned)(HD / kPvCols), (unsigned)KVH, (unsigned)((B + kPvTileRows - 1) / kPvTileRows));
     const int G = H / KVH;
     const unsigned nthr = (unsigned)(kPvTileRows * G * kPvCols);
@@ -2532,13 +2523,13 @@ void launch_attn_list_t(hipStream_t s, int HD, int B, int H, int KVH, const floa
 
 // kc, vc: fp32 caches, or fp16 ones when kv16.
 void launch_attn_list(hipStream_t s, int HD, int B, int H, int KVH, const float* qkv, int QKV, const void* kc,
-                      const void* vc, bool kv16, int ctx, int end, int layer, float* sc, float* att, int D, const int* pos,
+                      const void* vc, bool kv16, int ctx, AttnSpan sp, int layer, float* sc, float* att, int D, const int* pos,
                       size_t seq_stride, uint4* xq = nullptr, int xstride = 0, uint4* xh = nullptr) {
   if (kv16)
-    launch_attn_list_t<kvhalf>(s, HD, B, H, KVH, qkv, QKV, (const kvhalf*)kc, (const kvhalf*)vc, ctx, end, layer, sc, att,
+    launch_attn_list_t<kvhalf>(s, HD, B, H, KVH, qkv, QKV, (const kvhalf*)kc, (const kvhalf*)vc, ctx, sp, layer, sc, att,
                                D, pos, seq_stride, xq, xstride, xh);
   else
-    launch_attn_list_t<float>(s, HD, B, H, KVH, qkv, QKV, (const float*)kc, (const float*)vc, ctx, end, layer, sc, att, D,
+    launch_attn_list_t<float>(s, HD, B, H, KVH, qkv, QKV, (const float*)kc, (const float*)vc, ctx, sp, layer, sc, att, D,
                               pos, seq_stride, xq, xstride, xh);
 }
 
@@ -2567,9 +2558,11 @@ bool attn_list_ok(int H, int KVH, int HD, int ctx) {
   return true;
 }
 
-// One pass over M <= MT tokens at device position st->pos0 (forward_pass, kernels.c:306-415), which ends
-// at position `end` at most.
-void enqueue_pass(q4hip* h, int M, bool want_logits, int end) {
+// The positions of a pass of M tokens from pos on.
+AttnSpan pass_span(int pos, int M) { return {pos + M, pos + (M + 1) / 2}; }
+
+// One pass over M <= MT tokens at device position st->pos0 (forward_pass, kernels.c:306-415), within sp.
+void enqueue_pass(q4hip* h, int M, bool want_logits, AttnSpan sp) {
   const int D = h->D, F = h->F, HD = h->HD, QKV = h->QKV;
   hipStream_t s = h->stream;
   uint4* xh = M > 1 ? h->xh : nullptr;
@@ -2601,7 +2594,7 @@ void enqueue_pass(q4hip* h, int M, bool want_logits, int end) {
     prof_mark(h, Q4HIP_PROF_ATTN);
     bool quantized = false;                 // the list P.V kernel wrote xq (and xh) itself
     if (M > 1 && h->ascr && h->list_attn == 1) {
-      launch_attn_list(s, HD, M, h->H, h->KVH, h->qkv, QKV, h->kc, h->vc, h->kv16, h->ctx, end, l, h->ascr, h->att, D, h->tpos, 0,
+      launch_attn_list(s, HD, M, h->H, h->KVH, h->qkv, QKV, h->kc, h->vc, h->kv16, h->ctx, sp, l, h->ascr, h->att, D, h->tpos, 0,
                        h->xq, h->xstride, xh);
       quantized = true;
     } else if (M > 1 && h->ascr) {
@@ -2619,7 +2612,7 @@ void enqueue_pass(q4hip* h, int M, bool want_logits, int end) {
         k_attn_prefill<128, float><<<ag, 256, 0, s>>>(h->qkv, QKV, h->H, h->KVH, (const float*)h->kc, (const float*)h->vc, h->ctx, l,
                                                       h->att, D, h->st, M, h->ascr);
     } else if (M == 1 && h->ascr && h->list_attn == 1) {
-      launch_attn_list(s, HD, 1, h->H, h->KVH, h->qkv, QKV, h->kc, h->vc, h->kv16, h->ctx, end, l, h->ascr, h->att, D, &h->st->pos0, 0,
+      launch_attn_list(s, HD, 1, h->H, h->KVH, h->qkv, QKV, h->kc, h->vc, h->kv16, h->ctx, sp, l, h->ascr, h->att, D, &h->st->pos0, 0,
                        h->xq, h->xstride, xh);
       quantized = true;
     } else if (HD == 64 && h->kv16) {
@@ -2829,8 +2822,9 @@ bool use_persistent(q4hip* h) {
   return h->pers_ok && !h->pers_broken;
 }
 
-// Attention of the multi-kernel path: the list kernels (scores over 64-position workgroups, softmax
-// and P.V per 32-column slice) when the shape admits them, with the [MT][H][ctx] score buffer.
+// Attention of the multi-kernel path: k_attn_head, k_attn_rows and the list kernels (scores over
+// 64-position workgroups, softmax and P.V per 32-column slice; launch_attn_list_t chooses) when the shape
+// admits them, with the [MT][H][ctx] score buffer.
 void prepare_attention(q4hip* h) {
   if (h->list_attn < 0) h->list_attn = attn_list_ok(h->H, h->KVH, h->HD, h->ctx) ? 1 : 0;
   if (!h->ascr && (h->list_attn == 1 || h->MT > 1)) {
@@ -2842,9 +2836,11 @@ void prepare_attention(q4hip* h) {
 }
 
 // In AUTO mode, when the persistent kernel cannot split attention over two workgroups per head (too
-// few CUs), decode steps whose context reaches this many positions run on the multi-kernel path: its
-// attention spreads the scores over many workgroups and reads each kv head's K once, where the
-// persistent kernel streams a kv head's K and V through one workgroup per query head.
+// few CUs), decode steps whose context reaches this many positions run on the multi-kernel path, whose
+// attention shares a head's positions among four waves that all load and add (k_attn_head).  Where they
+// meet depends on what keeps the split out; on a device that has it, with the split switched off
+// (Q4HIP_SPLIT_FROM), the 0.5B shape's step takes 0.96 ms on either at 768 positions (fp32 cache), 1.86
+// against 1.29 at 2,048, 2.58 against 1.61 here.
 constexpr int kLongDecodePositions = 3072;
 
 bool long_decode(const q4hip* h, int64_t last_pos) {
@@ -2915,8 +2911,16 @@ bool aborted(q4hip* h) {
   return true;
 }
 
-int build_graph(q4hip* h) {
-  if (h->graph || h->graph_failed) return Q4HIP_OK;
+// Which captured step takes the token at `pos`: 0 with k_attn_head, 1 with the list kernels (the same
+// one at every position for most shapes).
+int step_graph(const q4hip* h, int pos) {
+  return h->list_attn != 1 || head_takes_rows(1, h->H, h->KVH, h->HD, h->kv16, pass_span(pos, 1)) ? 0 : 1;
+}
+
+// Capture the step that takes the token at `pos`, unless it is there.
+int build_graph(q4hip* h, int pos) {
+  hipGraphExec_t* const graph = &h->graph[step_graph(h, pos)];
+  if (*graph || h->graph_failed) return Q4HIP_OK;
   const char* env = getenv("Q4HIP_GRAPH");
   if (env && env[0] == '0') {   // eager launches, e.g. under a tracer that cannot follow graphs
     h->graph_failed = true;
@@ -2928,21 +2932,29 @@ int build_graph(q4hip* h) {
     (void)hipGetLastError();
     return Q4HIP_OK;
   }
-  enqueue_pass(h, 1, true, h->ctx);
+  enqueue_pass(h, 1, true, {h->ctx, pass_span(pos, 1).mean});       // replayed at other positions
   hipError_t e = hipStreamEndCapture(h->stream, &g);
-  if (e == hipSuccess) e = hipGraphInstantiate(&h->graph, g, nullptr, nullptr, 0);
+  if (e == hipSuccess) e = hipGraphInstantiate(graph, g, nullptr, nullptr, 0);
   if (g) (void)hipGraphDestroy(g);
   if (e != hipSuccess) {
-    h->graph = nullptr;
+    *graph = nullptr;
     h->graph_failed = true;
     (void)hipGetLastError();
   }
   return Q4HIP_OK;
 }
 
-void decode_step(q4hip* h) {
-  if (h->graph) (void)hipGraphLaunch(h->graph, h->stream);
-  else enqueue_pass(h, 1, true, h->ctx);
+void decode_step(q4hip* h, int pos) {
+  const hipGraphExec_t graph = h->graph[step_graph(h, pos)];
+  if (graph) (void)hipGraphLaunch(graph, h->stream);
+  else enqueue_pass(h, 1, true, pass_span(pos, 1));
+}
+
+void drop_graphs(q4hip* h) {
+  for (hipGraphExec_t& graph : h->graph) {
+    if (graph) (void)hipGraphExecDestroy(graph);
+    graph = nullptr;
+  }
 }
 
 }  // namespace
@@ -2963,7 +2975,7 @@ void q4hip_destroy(q4hip* h) {
   if (!h) return;
   (void)hipSetDevice(h->device);
   if (h->stream) (void)hipStreamSynchronize(h->stream);
-  if (h->graph) (void)hipGraphExecDestroy(h->graph);
+  drop_graphs(h);
   for (Layer& y : h->L) {
     mat_free(y.qkv); mat_free(y.o); mat_free(y.gu); mat_free(y.down);
     if (y.attn_norm) (void)hipFree(y.attn_norm);
@@ -3109,10 +3121,7 @@ int q4hip_set_tensor(q4hip* h, int kind, int layer, int row0, int type, const vo
     if (type != Q4HIP_TYPE_Q4_0 && type != Q4HIP_TYPE_Q8_0) return fail(Q4HIP_ETYPE, "kind 8: expected Q4_0 or Q8_0");
     if (type != h->head.fmt) {
       if (h->head.loaded > 0) return fail(Q4HIP_ETYPE, "kind 8: rows of Q4_0 and Q8_0 mixed");
-      if (h->graph) {   // the captured pass holds the old head's addresses
-        (void)hipGraphExecDestroy(h->graph);
-        h->graph = nullptr;
-      }
+      drop_graphs(h);   // the captured pass holds the old head's addresses
       mat_free(h->head);
       const int rc = mat_alloc(h->head, h->V, h->D, h->stream, type);
       if (rc != Q4HIP_OK) return rc;
@@ -3151,7 +3160,7 @@ int q4hip_forward(q4hip* h, const int* ids, int n, int pos, int* next) {
   HIPCHK(hipSetDevice(h->device));
   prepare_attention(h);
   const bool pers = n == 1 && use_persistent(h) && !long_decode(h, pos);
-  if (n == 1 && !pers) build_graph(h);
+  if (n == 1 && !pers) build_graph(h, pos);
   memcpy(h->pin_ids, ids, (size_t)n * 4);
   HIPCHK(hipMemcpyAsync(h->tokens + pos, h->pin_ids, (size_t)n * 4, hipMemcpyHostToDevice, h->stream));
   for (int c = 0; c < n; c += h->MT) {
@@ -3161,11 +3170,11 @@ int q4hip_forward(q4hip* h, const int* ids, int n, int pos, int* next) {
     if (k == 1 && last && pers) {
       HIPCHK(launch_persistent(h, pos + c, 1));
       h->last_mode = Q4HIP_DECODE_PERSISTENT;
-    } else if (k == 1 && last && h->graph) {
-      HIPCHK(hipGraphLaunch(h->graph, h->stream));
+    } else if (k == 1 && last && h->graph[step_graph(h, pos + c)]) {
+      HIPCHK(hipGraphLaunch(h->graph[step_graph(h, pos + c)], h->stream));
       h->last_mode = Q4HIP_DECODE_GRAPH;
     } else {
-      enqueue_pass(h, k, last, pos + c + k);
+      enqueue_pass(h, k, last, pass_span(pos + c, k));
       if (k == 1) h->last_mode = Q4HIP_DECODE_GRAPH;
     }
   }
@@ -3249,7 +3258,10 @@ static int run_generate(q4hip* h, int first, int pos, int steps, int* out, float
   HIPCHK(hipSetDevice(h->device));
   prepare_attention(h);
   const bool pers = use_persistent(h) && !long_decode(h, (int64_t)pos + steps - 1);
-  if (!pers) build_graph(h);
+  if (!pers) {
+    build_graph(h, pos);
+    build_graph(h, pos + steps - 1);
+  }
   h->pin_ids[0] = first;
   HIPCHK(hipMemcpyAsync(h->tokens + pos, h->pin_ids, 4, hipMemcpyHostToDevice, h->stream));
   k_set_pos<<<1, 64, 0, h->stream>>>(h->st, pos);
@@ -3263,7 +3275,7 @@ static int run_generate(q4hip* h, int first, int pos, int steps, int* out, float
     HIPCHK(launch_persistent(h, pos, steps));
     h->last_mode = Q4HIP_DECODE_PERSISTENT;
   } else {
-    for (int i = 0; i < steps; i++) decode_step(h);
+    for (int i = 0; i < steps; i++) decode_step(h, pos + i);
     h->last_mode = Q4HIP_DECODE_GRAPH;
   }
   if (ms) HIPCHK(hipEventRecord(e1, h->stream));
@@ -3306,7 +3318,7 @@ int q4hip_profile_pass(q4hip* h, const int* ids, int ntok, int pos, float* us, i
   k_set_pos<<<1, 64, 0, h->stream>>>(h->st, pos);
   std::vector<std::pair<int, hipEvent_t>> marks;
   h->prof = &marks;
-  enqueue_pass(h, ntok, true, pos + ntok);
+  enqueue_pass(h, ntok, true, pass_span(pos, ntok));
   h->prof = nullptr;
   hipError_t e = hipStreamSynchronize(h->stream);
   for (int i = 0; i < Q4HIP_PROF_N; i++) us[i] = 0.0f;
@@ -3402,8 +3414,8 @@ struct q4hip_batch {
 namespace {
 
 // One decode step of all B sequences: tokens bt->tok at positions bt->pos; the greedy tokens go to
-// bt->tok (and out[0..B) when given) and every position advances by one, to `end` at most.
-void enqueue_batch_step(q4hip_batch* bt, int* out, int end) {
+// bt->tok (and out[0..B) when given) and every position advances by one, within sp.
+void enqueue_batch_step(q4hip_batch* bt, int* out, AttnSpan sp) {
   q4hip* h = bt->h;
   const int B = bt->B, D = h->D, F = h->F, HD = h->HD, QKV = h->QKV;
   hipStream_t s = h->stream;
@@ -3426,7 +3438,7 @@ void enqueue_batch_step(q4hip_batch* bt, int* out, int end) {
                                                                         (float*)bt->kc, (float*)bt->vc, h->ctx, l,
                                                                         bt->pos, bt->seq_stride);
     }
-    launch_attn_list(s, HD, B, h->H, h->KVH, h->qkv, QKV, bt->kc, bt->vc, h->kv16, h->ctx, end, l, bt->sc, h->att, D, bt->pos,
+    launch_attn_list(s, HD, B, h->H, h->KVH, h->qkv, QKV, bt->kc, bt->vc, h->kv16, h->ctx, sp, l, bt->sc, h->att, D, bt->pos,
                      bt->seq_stride, h->xq, h->xstride, xh);
     launch_matvec<OP_ADD>(s, y.o, h->xq, h->xstride, B, h->x, D, nullptr, xh);
     launch_quant<QM_NORM>(s, B, h->x, D, D, y.ffn_norm, h->eps, h->xq, h->xstride, 0, xh);
@@ -3548,7 +3560,7 @@ int q4hip_batch_prefill(q4hip_batch* bt, int seq, const int* ids, int n, int pos
   for (int c = 0; e == hipSuccess && c < n; c += h->MT) {
     const int k = std::min(h->MT, n - c);
     k_set_pos<<<1, 64, 0, h->stream>>>(h->st, pos + c);
-    enqueue_pass(h, k, c + k >= n, pos + c + k);
+    enqueue_pass(h, k, c + k >= n, pass_span(pos + c, k));
   }
   h->kc = kc;
   h->vc = vc;
@@ -3589,8 +3601,10 @@ static int run_batch(q4hip_batch* bt, const int* first, const int* pos, int step
     HIPCHK(hipEventCreate(&e1));
     HIPCHK(hipEventRecord(e0, h->stream));
   }
-  const int end = *std::max_element(pos, pos + B) + steps;
-  for (int i = 0; i < steps; i++) enqueue_batch_step(bt, bt->out + (size_t)i * B, end);
+  int64_t sum = 0;
+  for (int b = 0; b < B; b++) sum += pos[b];
+  const AttnSpan sp = {*std::max_element(pos, pos + B) + steps, (int)(sum / B) + (steps + 1) / 2};
+  for (int i = 0; i < steps; i++) enqueue_batch_step(bt, bt->out + (size_t)i * B, sp);
   if (ms) HIPCHK(hipEventRecord(e1, h->stream));
   HIPCHK(hipGetLastError());
   HIPCHK(hipStreamSynchronize(h->stream));

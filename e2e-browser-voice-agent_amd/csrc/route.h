@@ -42,4 +42,69 @@ constexpr size_t attn_head_lds(int HD, int end) {
   return (size_t)kHeadStageBytes + (size_t)(head_row(end) + 16 + 4 * HD) * sizeof(float);
 }
 
+// The positions a call's rows look at: one past the last of any row, and a row's mean.
+struct AttnSpan {
+  int end, mean;
+};
+
+constexpr int kXcds = 8, kCus = 256;
+
+// k_attn_head's workgroups: units (row, kv head) dealt to the 8 XCDs, the G heads of a unit 8 apart.
+constexpr int attn_head_grid(int rows, int KVH, int G) { return (rows * KVH + kXcds - 1) / kXcds * kXcds * G; }
+
+// How many of its workgroups run at once.
+constexpr int head_slots(int HD, int end) { return kCus * (attn_head_lds(HD, end) <= 80 * 1024 ? 2 : 1); }
+
+// Whether k_attn_head takes a prompt pass of `rows` rows, against k_attn_rows (head_dim 64) or three
+// launches (128), which read a K row once for the heads of a group.  Both sides timed as whole passes, ms
+// theirs / its (0.5B shape: 14 heads of 64 in groups of 7; 1.5B shape: 12 of 128 in groups of 6):
+//   head_dim 64   while its workgroups run at once, any group and position (0.5B, 36 rows at 0 1.44 / 1.23,
+//     at 3,000 3.09 / 2.19).  A second round costs as much again, where k_attn_rows' time grows with the
+//     group: groups of 3 to 5 leave nothing (40 rows of groups of 4 at 600 1.68 / 1.72), larger ones half
+//     of it (0.5B, 48 rows at 3,000 3.11 / 2.88) and all of it while positions are few (72 rows at 220 1.73 /
+//     1.66, 600 1.94 / 1.93, 1,500 2.45 / 2.51), groups of two half (40 rows at 1,500 2.48 / 2.29, 62 at
+//     600 1.96 / 1.99).  No group: faster at any size measured, to 1,024 heads.
+//   head_dim 128  two rounds (1.5B, fp16, 64 rows at 3,000 5.93 / 5.21), with fp32 rows up to some 1,400
+//     positions (64 rows at 1,000 4.16 / 3.98, 72 at 1,500 4.84 / 4.90, 48 at 3,000 5.72 / 5.81); more where
+//     positions are few (fp32, 128 rows at 220 4.54 / 4.46, at 400 4.73 / 4.77, 256 at 0 6.89 / 6.79, at 220
+//     7.28 / 7.57); groups of one or two at any size measured, to 3,072 heads.
+inline bool head_takes_pass(int rows, int H, int KVH, int HD, bool kv16, AttnSpan sp) {
+  const int G = H / KVH, slots = head_slots(HD, sp.end), grid = attn_head_grid(rows, KVH, G);
+  const int rounds = (grid + slots - 1) / slots;
+  if (rows * H > (HD == 64 ? 1024 : 3072)) return false;
+  if (rounds == 1 || G == 1) return true;
+  if (HD == 64) {
+    if (slots == kCus) return G >= 6 && rounds == 2;       // 0.5B, 32 rows at 3,600: 79 / 65 us a layer
+    return G == 2 ? grid <= 768 : G >= 6 && (grid <= 768 || (rounds == 2 && sp.mean <= 704));
+  }
+  if (G == 2) return true;
+  return rounds == 2 ? kv16 || sp.mean <= 1400 : (long)rounds * sp.mean <= (kv16 ? 1700 : 1350);
+}
+
+// Whether it takes one token, or one of each sequence of a batch, against k_attn_scores_list and
+// k_attn_pv_list, which spread a row's positions over workgroups and read a cache row once for the heads
+// of a group.  ms of a whole step, theirs / its (32 sequences of 300, 0.5B 1.63 / 1.40).  Not:
+//   * rows of 128 fp32 columns past some positions.  The heads of a group read the rows one after the
+//     other, and from there on the rows leave the L2 in between.  1.5B, 2 sequences of 700 2.47 / 2.39, of
+//     1,024 2.59 / 2.68; 32 of 700 2.83 / 2.75, of 3,000 4.09 / 4.83; one token of 12 layers at 700 0.71 /
+//     0.67, at 1,500 0.83 / 0.91; the smaller the group, the sooner (16 heads in groups of 4, 2 sequences of
+//     600 1.007 times as fast, of 1,024 0.94; in groups of 1 300 1.00, 1,024 0.86).  Large batches of small
+//     groups read enough on either side to hide it (groups of 4, 24 sequences of 3,000 1.05; groups of 2, 16
+//     sequences 1.05).
+//   * large groups in more workgroups than run at once: head_dim 64 past some 600 or 700 positions
+//     (0.5B, 64 sequences of 500 1.92 / 1.88, of 700 2.00 / 2.06, 48 of 700 1.85 / 1.83), and past some 3,500, where one workgroup fits a CU (32
+//     sequences of 3,800 83 / 91 us a layer).
+inline bool head_takes_rows(int rows, int H, int KVH, int HD, bool kv16, AttnSpan sp) {
+  const int G = H / KVH, slots = head_slots(HD, sp.end), grid = attn_head_grid(rows, KVH, G);
+  const int rounds = (grid + slots - 1) / slots;
+  if (HD == 128 && !kv16) {
+    const int most = G >= 5 ? (rounds == 1 ? 832 : 640) : G >= 3 ? 704 : G == 2 ? 512 : 384;
+    const bool many = G <= 2 ? grid >= 128 * G : G == 4 && grid >= 384;
+    if (sp.mean > most && !(many && slots == 2 * kCus)) return false;
+  }
+  if (rounds == 1 || G <= 2) return true;
+  if (slots == kCus) return false;
+  return HD == 128 || G <= 4 || sp.mean <= (grid <= 768 ? 704 : 576);
+}
+
 }  // namespace q4

@@ -77,6 +77,46 @@ def test_sum_by_the_wave(name, kv):
         o.close()
 
 
+def test_steps_across_the_limit_of_fp32_rows():
+    """Two heads of 128 fp32 columns in one group: a token, and a small batch by its mean, takes this
+    kernel up to 512 positions and the list kernels from there (the token in two captured steps)."""
+    import q4hip
+    shape, g, o = _pair("small128", "f32", 1000)
+    try:
+        ids = synth.prompt_ids(9, 506, shape.vocab)
+        want = [o.forward(ids, 0)]
+        for i in range(14):
+            want.append(o.forward([want[-1]], 506 + i))
+        last = o.logits().copy()
+        assert g.forward(ids, 0) == want[0]
+        for run in range(3):                         # the second and third run replay both graphs
+            print(f"generate, run {run}", flush=True)
+            assert g.generate(want[0], 506, 14) == want[1:]
+            _same(g.read_logits(), last, f"run {run}")
+        for i in range(14):
+            assert g.forward([want[i]], 506 + i) == want[i + 1], f"token {i}"
+        _same(g.read_logits(), last, "token by token")
+        lens = [505, 500, 511]                       # means of 507 (2 steps) and 520
+        bt = q4hip.Batch(g, 3)
+        try:
+            ps = [synth.prompt_ids(40 + n, n, shape.vocab) for n in lens]
+            first = [bt.prefill(b, ps[b], 0) for b in range(3)]
+            a = bt.generate(first, lens, 2)
+            c = bt.generate(a[-1], [n + 2 for n in lens], 25)
+            lg = bt.read_logits()
+        finally:
+            bt.close()
+        for b, n in enumerate(lens):
+            w = [o.forward(ps[b], 0)]
+            for i in range(27):
+                w.append(o.forward([w[-1]], n + i))
+            assert [first[b]] + a[:, b].tolist() + c[:, b].tolist() == w, f"sequence of {n}"
+            _same(lg[b], o.logits(), f"sequence of {n}")
+    finally:
+        g.close()
+        o.close()
+
+
 def test_time_follows_the_positions_not_the_context():
     """36 rows of 14 heads are 504 workgroups: two fit a CU with the shared memory of 36 positions, one with
     that of a 4,400-position context (attention 1.5 times as long).  Best of 9 in turn; 1.25 is half way."""
