@@ -1782,7 +1782,7 @@ int check_ready(q4hip* h) {
 // Kernel choice for passes of M > 1 tokens (every candidate gives the same bits):
 //   k_gemm_sk (matrix cores, operands streamed through a shared-memory ring), one lane chain per
 //   wave (JS 4) when the matrix has too few rows to give 512 workgroups of 64 rows, else all four
-//   chains per wave (JS 1); k_gemm_tile for large passes (tile_fills).  Measured on MI355X against the earlier matrix-core GEMM with register
+//   chains per wave (JS 1); k_gemm_tile for large passes (tile_takes).  Measured on MI355X against the earlier matrix-core GEMM with register
 //   prefetch: 1024-token prefill 15.0 -> 10.5 ms, 32-sequence batched step 4.3 -> 3.7 ms.
 //   From 2 tokens on: most of the 16-token tile is then idle, but a projection is bound by its
 //   chain of blocks, not by its columns.  The one-token kernel run over 2..8 tokens of activations
@@ -1800,31 +1800,9 @@ bool sk_enabled() {
   return on;
 }
 
-// Whether k_gemm_tile (64 tokens x 32 rows) takes a projection of `wgs` workgroups.  Its time steps up
-// with every round of 256 workgroups (one, two, three on a CU: down of the 0.5B shape 47, 59 us for up
-// to 256, 512), where k_gemm_sk's grows with the tokens (34 us at 331, 76 us at 1,024), so it takes the
-// sizes that nearly fill their last round.  Measured on whole passes, all projections but gate|up
-// through it against none: 1.5B shape 1,000 tokens 22.4 / 23.3 ms, 640 15.0 / 15.4, 320 9.26 / 9.47,
-// but 512 (384 workgroups for o and down) 12.8 / 12.3; 0.5B shape 1,000 8.44 / 8.61, 768 6.86 / 6.50.
-constexpr int kTileMinTokens = 256;   // below, half of a 64-token tile may be idle
-inline bool tile_fills(int wgs) {
-  const int rounds = (wgs + 255) / 256, percent = wgs * 100 / (256 * rounds);
-  return percent >= (rounds == 1 ? 90 : rounds == 2 ? 85 : 75);
-}
-
-// Whether k_gemm_tile (64 tokens x one 32-value block) takes the fused gate|up projection of nrg blocks:
-// from about two workgroups per CU on; up to three token tiles only where the last one is more than half
-// full.  Whole passes through it / through k_gemm_sk: 0.5B shape 128 tokens 2.05 / 1.95 ms, 192 2.36 /
-// 2.48, 512 4.35 / 4.80, 1,000 7.65 / 8.61; 1.5B shape 128 4.15 / 4.21, 160 5.30 / 5.17, 192 5.83 /
-// 6.05, 1,000 20.4 / 23.3.
-inline bool tile_gu(int nrg, int M) {
-  const int nt = (M + 63) / 64;
-  return nrg * nt >= 456 && (nt > 3 || (M - 1) % 64 >= 32);
-}
-
-int pick_gemm(const Mat& W, int M, bool have_xh) {
-  if (have_xh && sk_enabled() && W.nb % 4 == 0 && M >= kTileMinTokens && tile_fills(W.Np / 32 * ((M + 63) / 64)))
-    return GK_TILE;
+// qkv: the q|k|v projection, the only one with a bias.
+int pick_gemm(const Mat& W, int M, bool have_xh, bool qkv) {
+  if (have_xh && sk_enabled() && W.nb % 4 == 0 && tile_takes(W.Np / 32, M, qkv)) return GK_TILE;
   if (have_xh && sk_enabled() && W.nb % 4 == 0)            // k_gemm_sk takes whole groups of 4 blocks
     return (W.Np / 64) * ((M + 15) / 16) >= 512 ? GK_SK1 : GK_SK4;
   if (M <= 64) return M >= 16 ? GK_ROWS2 : GK_ROWS1;
@@ -1867,7 +1845,7 @@ void launch_tile(hipStream_t s, const Mat& W, int nrg, const uint4* xh, int xstr
 bool launch_gu_swiglu(hipStream_t s, const Mat& W, const uint4* xh_in, int xstride, int M, uint4* xq_out,
                       uint4* xh_out, int F) {
   if (!xh_in || F % 32 || !sk_enabled() || W.nb % 4) return false;
-  if (tile_gu(F / 32, M)) {
+  if (tile_takes_gu(F / 32, M)) {
     launch_tile<OP_STORE, 1, 1>(s, W, F / 32, xh_in, xstride, M, nullptr, 0, nullptr, xq_out, xh_out, F);
     return true;
   }
@@ -1884,7 +1862,7 @@ bool launch_gu_swiglu(hipStream_t s, const Mat& W, const uint4* xh_in, int xstri
 bool launch_qkv_rope(hipStream_t s, const Mat& W, const uint4* xh, int xstride, int M, float* qkv, int QKV,
                      const float* bias, const SkRope& rp) {
   if (!xh || rp.hd % 32) return false;
-  const int kind = pick_gemm(W, M, true);
+  const int kind = pick_gemm(W, M, true, true);
   if (kind == GK_TILE) {
     launch_tile<OP_BIAS, 2, 2>(s, W, W.Np / 32, xh, xstride, M, qkv, QKV, bias, nullptr, nullptr, 0, rp);
     return true;
@@ -1922,7 +1900,7 @@ template <int OP>
 void launch_matvec(hipStream_t s, const Mat& W, const uint4* xq, int xstride, int M, float* y, int ldy,
                    const float* bias, const uint4* xh = nullptr) {
   if (M == 1) return launch_matvec1<OP>(s, W, xq, y, bias);
-  switch (pick_gemm(W, M, xh != nullptr)) {
+  switch (pick_gemm(W, M, xh != nullptr, OP == OP_BIAS)) {
     case GK_ROWS2: launch_rows<OP, 2>(s, W, xq, xstride, M, y, ldy, bias); break;
     case GK_ROWS1: launch_rows<OP, 1>(s, W, xq, xstride, M, y, ldy, bias); break;
     case GK_TILE: launch_tile<OP, 2, 0>(s, W, W.Np / 32, xh, xstride, M, y, ldy, bias); break;

@@ -6,6 +6,8 @@
 
 namespace q4 {
 
+constexpr int kXcds = 8, kCus = 256;
+
 // ---- one-token projections
 
 // k_matvec_split takes rows of kSplitMinBlocks .. kSplitMaxBlocks blocks.
@@ -29,6 +31,40 @@ inline bool mv_quantizes_itself(int N, int nb) {
   return wgs <= 1792 && wgs * nb <= 440000;
 }
 
+// ---- projections of prompt passes
+
+// Whether k_gemm_tile (64 tokens x 32 rows, three workgroups on a CU) takes a projection of nrg groups of 32
+// rows, against k_gemm_sk; qkv: the q|k|v projection, whose epilogue is RoPE and the cache append.  Its
+// time steps up with every round of 256 workgroups (down of the 0.5B shape 47 us in one round, 59 in two),
+// where k_gemm_sk's grows with every 16 tokens, so it takes the sizes that nearly fill their last round: a
+// single round by the 16-token groups it holds, more by the workgroups.  Whole passes, ms by k_gemm_sk / with
+// o and down by k_gemm_tile:
+//   one round     1.5B shape 288 tokens 7.25 / 7.50, 304 7.57 / 7.57, 320 7.68 / 7.67; 0.5B 512 4.21 / 4.30,
+//                 544 4.75 / 4.73
+//   two, three..  1.5B 512 9.72 / 10.31, 608 12.03 / 11.65, 672 13.2 / 13.7, 768 14.83 / 14.79, 1,024 19.3 /
+//                 18.4; 0.5B 640 4.97 / 5.33, 864 6.35 / 6.69, 992 7.55 / 7.38
+// q|k|v in one or two rounds is slower with its registers' RoPE epilogue (0.5B 448 tokens 4.13 / 4.18, 832
+// 6.10 / 6.18, 1.5B 400 8.85 / 8.90) and level from there (1.5B 576 11.56 / 11.61, 1,024 19.26 / 19.10).
+constexpr int kTileMinTokens = 256;   // below, half of a 64-token tile may be idle
+inline bool tile_takes(int nrg, int M, bool qkv) {
+  if (M < kTileMinTokens) return false;
+  const int wgs = nrg * ((M + 63) / 64), rounds = (wgs + kCus - 1) / kCus;
+  if (rounds <= 2 && qkv) return false;
+  if (rounds == 1) return nrg * ((M + 15) / 16) * 100 >= 88 * 4 * kCus;
+  return wgs * 100 >= (rounds == 2 ? 85 : 75) * kCus * rounds;
+}
+
+// Whether it takes the fused gate|up projection (64 tokens x one 32-value block) of nrg blocks: from nearly
+// two workgroups per CU on (456: 152 blocks by three tiles was the least that paid, 304 the most that did
+// not), up to three token tiles only where the last one is well filled.  Whole passes, ms by k_gemm_sk / by
+// it: 0.5B shape 128 tokens 1.84 / 1.91, 160 2.15 / 2.14, 176 2.31 / 2.23, 193 2.42 / 2.40, 208 2.44 / 2.42,
+// 224 2.73 / 2.64, 257 3.03 / 2.82; 1.5B 112 3.83 / 3.90, 120 4.15 / 4.10, 160 4.99 / 5.18, 176 5.63 / 5.61, 193
+// 6.08 / 5.92, 224 6.72 / 6.43, 288 8.02 / 7.49.
+inline bool tile_takes_gu(int nrg, int M) {
+  const int nt = (M + 63) / 64, last = M - 64 * (nt - 1);
+  return nrg * nt >= 456 && last > (nt <= 2 ? 48 : nt == 3 ? 32 : 0);
+}
+
 // ---- attention
 
 // Shared memory of k_attn_head, whose workgroup takes one row and head: the K stages and V slots, the row
@@ -46,8 +82,6 @@ constexpr size_t attn_head_lds(int HD, int end) {
 struct AttnSpan {
   int end, mean;
 };
-
-constexpr int kXcds = 8, kCus = 256;
 
 // k_attn_head's workgroups: units (row, kv head) dealt to the 8 XCDs, the G heads of a unit 8 apart.
 constexpr int attn_head_grid(int rows, int KVH, int G) { return (rows * KVH + kXcds - 1) / kXcds * kXcds * G; }

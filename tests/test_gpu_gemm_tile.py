@@ -1,6 +1,7 @@
 """The 32 x 32 matrix-core tiles of large prompt passes against the oracle: token counts at the edges of the
-16-, 32- and 64-token tiles, on shapes wide enough that the projections (hidden 2048, with the RoPE
-epilogue at head_dim 64 and 128) or the fused gate|up projection (ffn 8192) take them.  Tokens equal,
+16-, 32- and 64-token tiles, on shapes wide enough that the projections (hidden 2048: o and down at 256 and
+from 385 tokens, with the RoPE epilogue at head_dim 64 and 128 from 449) or the fused gate|up projection (ffn
+8192, from 113) take them; the other counts stay on k_gemm_sk.  Tokens equal,
 logits bit for bit; a decode step after each pass reads the caches that the pass wrote.
 """
 import numpy as np
@@ -12,9 +13,10 @@ import synth
 pytestmark = pytest.mark.gpu
 
 CASES = {  # shape (the oracle takes hidden up to ffn), token counts
-    "hd64": (synth.Shape(2048, 1, 2048, 32, 4, 512), (256, 321, 336, 337, 353, 369, 384, 450, 512)),
-    "hd128": (synth.Shape(2048, 1, 2048, 16, 2, 512), (256, 330, 352, 384, 500)),
-    "gate_up": (synth.Shape(128, 1, 8192, 2, 1, 512), (97, 127, 128, 161, 193, 208, 209, 225, 240, 256, 257)),
+    "hd64": (synth.Shape(2048, 1, 2048, 32, 4, 512), (256, 321, 336, 337, 353, 369, 384, 400, 417, 449,
+                                                           450, 464, 465, 481, 497, 512)),
+    "hd128": (synth.Shape(2048, 1, 2048, 16, 2, 512), (256, 330, 352, 384, 385, 449, 481, 500)),
+    "gate_up": (synth.Shape(128, 1, 8192, 2, 1, 512), (97, 113, 127, 128, 161, 193, 208, 209, 225, 240, 256, 257)),
 }
 
 
