@@ -2516,7 +2516,10 @@ void launch_attn_list(hipStream_t s, int HD, int B, int H, int KVH, const float*
 bool attn_list_ok(int H, int KVH, int HD, int ctx) {
   if (H / KVH > kMaxGroup) return false;
   int dev = 0;
-  if (hipGetDevice(&dev) == hipSuccess) (void)(attn_rows_setup(dev) && attn_head_setup(dev));
+  if (hipGetDevice(&dev) == hipSuccess) {
+    (void)attn_rows_setup(dev);
+    (void)attn_head_setup(dev);
+  }
   const size_t lds = attn_pv_lds(H, KVH, ctx), slds = softmax_lds(H, KVH, ctx);
   if (lds > 160 * 1024) return false;
   if (slds > 64 * 1024 &&
