@@ -54,3 +54,36 @@ def test_passes_and_batches_of_a_few_tokens(name, head):
     finally:
         g.close()
         o.close()
+
+
+@pytest.mark.parametrize("shape", [synth.Shape(128, 1, 256, 2, 1, 192), synth.Shape(192, 1, 256, 3, 1, 1090),
+                                   synth.Shape(2112, 1, 2112, 33, 11, 192)], ids=["vocab192", "vocab1090", "hidden2112"])
+def test_q8_head_of_batches(shape):
+    """The Q8_0 head for several tokens: an odd number of 64-row tiles (192), rows that end inside one
+    (1,090), rows wider than it takes (2,112 values: a launch per sequence), and batches at the edges of the 4,
+    8 and 16 tokens of a workgroup."""
+    import q4hip
+    t = synth.make_model(shape, 93, head_type=synth.GGML_Q8_0)
+    g = q4hip.Model(shape, ctx=48)
+    g.load(t)
+    o = oracle.Model(shape, t, ctx=48, mt=16, threads=8)
+    try:
+        for B in (1, 2, 4, 5, 8, 9, 16, 17, 33):
+            print(f"vocab {shape.vocab} hidden {shape.dim} batch of {B}", flush=True)
+            lens = [1 + (5 * b) % 7 for b in range(B)]
+            ps = [synth.prompt_ids(20 + b, n, shape.vocab) for b, n in enumerate(lens)]
+            bt = q4hip.Batch(g, B)
+            try:
+                first = [bt.prefill(b, ps[b], 0) for b in range(B)]
+                out = bt.generate(first, lens, 1)
+                lg = bt.read_logits()
+            finally:
+                bt.close()
+            for b in range(B):
+                want = o.forward(ps[b], 0)
+                assert first[b] == want, f"batch of {B}, sequence {b}"
+                assert out[0, b] == o.forward([want], lens[b]), f"batch of {B}, sequence {b}"
+                _same(lg[b], o.logits(), f"batch of {B}, sequence {b}")
+    finally:
+        g.close()
+        o.close()
