@@ -449,8 +449,10 @@ __device__ __forceinline__ int dpp_or_0(int v) {
 // against 3,400, 1,026 values 8,700 against 8,600, 4,097 values 9,000 against 32,000.
 constexpr int kOrderedWaveMin = 1280;
 
-// Called by all 64 lanes of a wave (T >= 1, every value >= +0); the sum, the same in every lane.
-__device__ __forceinline__ float ordered_sum_wave(const float* e, int T) {
+// Called by all 64 lanes of a wave (T >= 1, every value >= +0); the sum, the same in every lane.  With
+// `combined`, whether the runs were combined (an assumption may fail, and short sums are not worth it).
+__device__ __forceinline__ float ordered_sum_wave(const float* e, int T, bool* combined = nullptr) {
+  if (combined) *combined = false;
   if (T < kOrderedWaveMin) return ordered_sum(e, T);
   const int lane = (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
   const int R = ordered_run(T), n = (T + R - 1) / R;     // n <= 64 runs
@@ -537,6 +539,7 @@ __device__ __forceinline__ float ordered_sum_wave(const float* e, int T) {
   }
   segment(n);
   if (!ok) return ordered_sum(e, T);
+  if (combined) *combined = true;
   return __int_as_float(S);
 }
 

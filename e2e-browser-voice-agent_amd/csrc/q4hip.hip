@@ -3831,7 +3831,7 @@ int q4hip_mv_run_noalloc(q4hip_mv* m, const float* x, float* y, void* stream) {
 
 }  // extern "C"
 
-// ---------------------------------------------------------------- quotient self-check
+// ---------------------------------------------------------------- self-checks: quotients, sums in order
 
 namespace {
 
@@ -3865,6 +3865,23 @@ __global__ __launch_bounds__(256) void k_check_division(int mode, uint32_t lo, u
   if (n) atomicAdd(bad + mode, n);
 }
 
+// The sums of row blockIdx.x, one wave per row, from shared memory laid out as k_attn_head's row of
+// exponentials: by the wave and by one lane.
+__global__ __launch_bounds__(64) void k_check_sum(const float* __restrict__ v, int n, float* __restrict__ wave,
+                                                  float* __restrict__ lane, int* __restrict__ combined) {
+  extern __shared__ __attribute__((aligned(16))) float lsm[];
+  for (int t = threadIdx.x; t < head_row(n); t += 64) lsm[t] = t < n ? v[(size_t)blockIdx.x * n + t] : 0.0f;
+  __syncthreads();
+  bool c;
+  const float s = ordered_sum_wave(lsm, n, &c), one = ordered_sum(lsm, n);
+  if (threadIdx.x == 0) {
+    wave[blockIdx.x] = s;
+    lane[blockIdx.x] = one;
+    combined[blockIdx.x] = c;
+  }
+}
+constexpr int kCheckSumMax = 15360;    // its row in 64 KB
+
 }  // namespace
 
 extern "C" {
@@ -3889,6 +3906,28 @@ int q4hip_check_division(int device, unsigned long long* mismatches, int n) {
   if (e == hipSuccess) e = hipMemcpy(mismatches, d, (size_t)n * sizeof(unsigned long long), hipMemcpyDeviceToHost);
   (void)hipFree(d);
   if (e != hipSuccess) return fail(Q4HIP_EHIP, "division check: %s", hipGetErrorString(e));
+  return Q4HIP_OK;
+}
+
+int q4hip_check_ordered_sum(int device, const float* v, int rows, int n, float* wave, float* lane, int* combined) {
+  if (!v || !wave || !lane || !combined) return fail(Q4HIP_EINVAL, "null argument");
+  if (rows < 1 || rows > 65535 || n < 1 || n > kCheckSumMax)
+    return fail(Q4HIP_EINVAL, "%d rows of %d values: 1..65535 of 1..%d", rows, n, kCheckSumMax);
+  HIPCHK(hipSetDevice(device));
+  const size_t bytes = (size_t)rows * n * 4, out = (size_t)rows * 4;
+  char* d = nullptr;
+  HIPCHK(hipMalloc(&d, bytes + 3 * out));
+  float* const w = (float*)(d + bytes);
+  hipError_t e = hipMemcpy(d, v, bytes, hipMemcpyHostToDevice);
+  if (e == hipSuccess) {
+    k_check_sum<<<rows, 64, (size_t)head_row(n) * 4>>>((const float*)d, n, w, w + rows, (int*)(w + 2 * (size_t)rows));
+    e = hipGetLastError();
+  }
+  if (e == hipSuccess) e = hipMemcpy(wave, w, out, hipMemcpyDeviceToHost);
+  if (e == hipSuccess) e = hipMemcpy(lane, w + rows, out, hipMemcpyDeviceToHost);
+  if (e == hipSuccess) e = hipMemcpy(combined, w + 2 * (size_t)rows, out, hipMemcpyDeviceToHost);
+  (void)hipFree(d);
+  if (e != hipSuccess) return fail(Q4HIP_EHIP, "sum check: %s", hipGetErrorString(e));
   return Q4HIP_OK;
 }
 

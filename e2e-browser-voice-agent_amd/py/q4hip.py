@@ -32,7 +32,7 @@ EXPORTS = [
     "q4hip_set_kv", "q4hip_profile_pass", "q4hip_batch_create", "q4hip_batch_destroy",
     "q4hip_batch_prefill", "q4hip_batch_set_kv", "q4hip_batch_generate", "q4hip_batch_time_generate",
     "q4hip_batch_read_logits", "q4hip_mv_time_cold", "q4hip_check_division", "q4hip_mv_run_noalloc",
-    "q4hip_attn_ring_rows",
+    "q4hip_attn_ring_rows", "q4hip_check_ordered_sum",
 ]
 
 _lib = None
@@ -56,6 +56,7 @@ def lib() -> ctypes.CDLL:
         "q4hip_last_error": (ctypes.c_char_p, []),
         "q4hip_device_count": (I, [ctypes.POINTER(I)]),
         "q4hip_check_division": (I, [I, P, I]),
+        "q4hip_check_ordered_sum": (I, [I, P, I, I, P, P, P]),
         "q4hip_create": (I, [ctypes.POINTER(P), I, I, I, I, I, I, I, I, F, I, I]),
         "q4hip_set_tensor": (I, [P, I, I, I, I, P, I64, ctypes.c_size_t]),
         "q4hip_set_rope": (I, [P, P, I64]),
@@ -133,6 +134,16 @@ def check_division(device: int = 0) -> dict:
     out = np.zeros(len(DIVISION_FORMS), np.uint64)
     _check(lib().q4hip_check_division(device, _ptr(out), len(DIVISION_FORMS)))
     return dict(zip(DIVISION_FORMS, (int(v) for v in out)))
+
+
+def check_ordered_sum(v: np.ndarray, device: int = 0) -> tuple:
+    """(sums by the wave, sums by one lane, whether the wave combined its runs) of the rows of v
+    (q4hip_check_ordered_sum)."""
+    v = np.ascontiguousarray(v, np.float32)
+    rows, n = v.shape
+    wave, lane, combined = np.empty(rows, np.float32), np.empty(rows, np.float32), np.empty(rows, np.int32)
+    _check(lib().q4hip_check_ordered_sum(device, _ptr(v), rows, n, _ptr(wave), _ptr(lane), _ptr(combined)))
+    return wave, lane, combined != 0
 
 
 def attn_ring_rows(pos: int, kv_tile: int, ring_slots: int, split: bool, half: int, kv_f16: bool) -> tuple:

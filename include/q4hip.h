@@ -116,7 +116,11 @@ int q4hip_generate(q4hip* h, int first, int pos, int steps, int* out);
 
 /* Per-operation GPU time of one decode step (forward([token], pos)), in microseconds, summed
  * over layers: profile (engine/cpu-worker.js:31-37, engine/kernels.c:481-483).  us[] receives
- * Q4HIP_PROF_N entries in the order of the Q4HIP_PROF_* indices. */
+ * Q4HIP_PROF_N entries in the order of the Q4HIP_PROF_* indices.  An operation that a projection's
+ * launch includes counts there: RMSNorm and quantize of a token's rows of 28 or 48 blocks, RoPE and
+ * the cache append under QKV, RMSNorm and SwiGLU with its quantize under GU, a quantize that the
+ * attention kernel writes itself under ATTN.  NORM_Q, ROPE, SWIGLU and QUANT then hold what is left
+ * (the output norm, the gaps between events). */
 #define Q4HIP_PROF_EMBED 0
 #define Q4HIP_PROF_NORM_Q 1
 #define Q4HIP_PROF_QKV 2
@@ -231,6 +235,14 @@ int q4hip_mv_run_noalloc(q4hip_mv* m, const float* x, float* y, void* stream);
  * [0] a / 127 (a >= 0), [1] d ? 1/d : 0 (d >= 0), [2] g / (1 + fast_exp(-g)) (every bit pattern),
  * [3] a / 896 (a >= 0), [4] 1 / d (d >= 0).  No counterpart in the reference (a diagnostic). */
 int q4hip_check_division(int device, unsigned long long* mismatches, int n);
+
+/* ---- self-check of the sums in order ---------------------------------------------------------
+ * The softmax sum adds its terms one after the other (engine/kernels.c:362-369); long ones are formed by a
+ * whole wave from runs it combines, with the same bits.  This sums each row of v (host memory, `rows`
+ * rows of n values >= +0, n up to 15360) on the device both ways: wave[] by the wave, lane[] by one
+ * lane, combined[] whether the wave combined its runs (rows past a length, no assumption failing).
+ * No counterpart in the reference (a diagnostic). */
+int q4hip_check_ordered_sum(int device, const float* v, int rows, int n, float* wave, float* lane, int* combined);
 
 /* ---- self-check of the attention ring's row bounds (host only, no GPU) ----------------------
  * The persistent decode kernel's attention workgroups stream past K/V rows through a ring in

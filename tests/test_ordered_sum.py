@@ -1,6 +1,7 @@
 """The wave's sum in order (ordered_sum_wave of csrc/kernels.h), restated in numpy float32 and compared bit
 for bit with the plain loop of additions: values near ties, exact powers of two, zeros, denormals, sums
-that sit on a power of two, one large value among small ones, infinities.
+that sit on a power of two, one large value among small ones, infinities.  The kernel itself runs the same kinds of
+values in tests/test_gpu_ordered_sum.py.
 """
 import numpy as np
 import pytest
