@@ -2025,8 +2025,9 @@ __device__ __forceinline__ bool attn_step(const PArgs& a, const PSmem& m, uint32
     lds_barrier();
     const float mpast = __builtin_fmaxf(__builtin_fmaxf(m.red[0], m.red[1]), __builtin_fmaxf(m.red[2], m.red[3]));
     // Long contexts: the past positions' sum by all of wave 0 (bit-identical, ordered_sum_wave), where
-    // ee has room for its padding.  8 steps after 4,096 positions 14.2 -> 13.0 ms.  The fp16-cache
-    // kernel only: in the fp32-cache one the code cost a short answer 0.9% without running.
+    // ee has room for its padding (not at the very end of a context of some 8,000 positions; there, and
+    // when the new score is the maximum, one lane adds).  8 steps after 4,096 positions 14.2 -> 13.0 ms.
+    // The fp16-cache kernel only: in the fp32-cache one the code cost a short answer 0.9% without running.
     const bool wsum = kF16 && pos >= kOrderedWaveMin && pos + ordered_run(pos) <= (int)attn_scores_floats(a.ctx);
     const int epad = wsum ? pos + ordered_run(pos) : (pos + 31) & ~31;
     for (int t = tid; t < epad; t += kPThreads) ee[t] = t < pos ? fast_exp(sc[t] - mpast) : 0.0f;

@@ -1782,8 +1782,9 @@ int check_ready(q4hip* h) {
 // Kernel choice for passes of M > 1 tokens (every candidate gives the same bits):
 //   k_gemm_sk (matrix cores, operands streamed through a shared-memory ring), one lane chain per
 //   wave (JS 4) when the matrix has too few rows to give 512 workgroups of 64 rows, else all four
-//   chains per wave (JS 1); k_gemm_tile for large passes (tile_takes).  Measured on MI355X against the earlier matrix-core GEMM with register
-//   prefetch: 1024-token prefill 15.0 -> 10.5 ms, 32-sequence batched step 4.3 -> 3.7 ms.
+//   chains per wave (JS 1); k_gemm_tile for large passes (tile_takes).  Measured on MI355X against the
+//   earlier matrix-core GEMM with register prefetch: 1024-token prefill 15.0 -> 10.5 ms, 32-sequence
+//   batched step 4.3 -> 3.7 ms.
 //   From 2 tokens on: most of the 16-token tile is then idle, but a projection is bound by its
 //   chain of blocks, not by its columns.  The one-token kernel run over 2..8 tokens of activations
 //   in global memory took 34.3 ms for 4 steps of 7 sequences of the 0.5B shape, k_gemm_rows 8.8 ms,
@@ -2020,7 +2021,7 @@ __global__ __launch_bounds__(256) void k_softmax_rows(float* __restrict__ sc, in
   }
 }
 
-// Q4HIP_PV_TILES=0 keeps prompt passes on k_attn_pv_list (same bits; for comparison).
+// Q4HIP_PV_TILES=0 keeps all attention on k_attn_scores_list and k_attn_pv_list (same bits; for comparison).
 bool pv_tiles_off() {
   static const bool off = [] { const char* e = getenv("Q4HIP_PV_TILES"); return e && e[0] == '0'; }();
   return off;

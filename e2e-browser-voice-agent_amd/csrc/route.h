@@ -125,9 +125,9 @@ inline bool head_takes_pass(int rows, int H, int KVH, int HD, bool kv16, AttnSpa
 //     600 1.007 times as fast, of 1,024 0.94; in groups of 1 300 1.00, 1,024 0.86).  Large batches of small
 //     groups read enough on either side to hide it (groups of 4, 24 sequences of 3,000 1.05; groups of 2, 16
 //     sequences 1.05).
-//   * large groups in more workgroups than run at once: head_dim 64 past some 600 or 700 positions
-//     (0.5B, 64 sequences of 500 1.92 / 1.88, of 700 2.00 / 2.06, 48 of 700 1.85 / 1.83), and past some 3,500, where one workgroup fits a CU (32
-//     sequences of 3,800 83 / 91 us a layer).
+//   * large groups in more workgroups than run at once: head_dim 64 past some 600 or 700 positions (0.5B,
+//     64 sequences of 500 1.92 / 1.88, of 700 2.00 / 2.06, 48 of 700 1.85 / 1.83), and past some 3,500
+//     positions, where one workgroup fits a CU (32 sequences of 3,800 83 / 91 us a layer).
 inline bool head_takes_rows(int rows, int H, int KVH, int HD, bool kv16, AttnSpan sp) {
   const int G = H / KVH, slots = head_slots(HD, sp.end), grid = attn_head_grid(rows, KVH, G);
   const int rounds = (grid + slots - 1) / slots;
