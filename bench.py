@@ -451,7 +451,7 @@ def bench_prefill(args):
         "config": {"workload": "qwen2.5-0.5b-shape Q4_0 prefill of 1024 seeded ids", "global_batch": 1,
                    "seq_len": n, "parallelism": "single-gpu"},
         "profile_us_per_pass": {k: round(v, 1) for k, v in prof.items()},
-        "roofline": {"bound": "mfma", "kernel": "whole prefill pass (projections on k_gemm_sk: exact block dots on the "
+        "roofline": {"bound": "mfma", "kernel": "whole prefill pass (projections on k_gemm_tile and k_gemm_sk: exact block dots on the "
                                                  "matrix cores, fp32 lane chains on the VALU)",
                      "achieved": round(pass_tflops, 2), "peak": 2500.0, "unit": "TFLOP/s (dense bf16 MFMA peak)",
                      "frac": round(pass_tflops / 2500.0, 5),
