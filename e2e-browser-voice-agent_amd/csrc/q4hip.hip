@@ -2444,7 +2444,7 @@ void launch_attn_list_t(hipStream_t s, int HD, int B, int H, int KVH, const floa
   const bool pass = seq_stride == 0 && B > 1;                // a prompt pass: rows share one cache
   if (xq && !pv_tiles_off() && !(pass && attn_rows_off()) &&
       (pass ? head_takes_pass(B, H, KVH, HD, sizeof(KT) == 2, sp)
-            : head_takes_rows(B, H, KVH, HD, sizeof(KT) == 2, sp)) &&
+            : head_takes_rows(B, H, KVH, HD, sizeof(KT) == 2, ctx, sp)) &&
       attn_head_lds(HD, sp.end) <= (size_t)kHeadMaxLds &&
       hipGetDevice(&dev) == hipSuccess && attn_head_setup(dev)) {
     const unsigned hg = attn_head_grid(B, KVH, Gq);
@@ -2539,9 +2539,6 @@ bool attn_list_ok(int H, int KVH, int HD, int ctx) {
   }
   return true;
 }
-
-// The positions of a pass of M tokens from pos on.
-AttnSpan pass_span(int pos, int M) { return {pos + M, pos + (M + 1) / 2}; }
 
 // One pass over M <= MT tokens at device position st->pos0 (forward_pass, kernels.c:306-415), within sp.
 void enqueue_pass(q4hip* h, int M, bool want_logits, AttnSpan sp) {
@@ -2896,7 +2893,7 @@ bool aborted(q4hip* h) {
 // Which captured step takes the token at `pos`: 0 with k_attn_head, 1 with the list kernels (the same
 // one at every position for most shapes).
 int step_graph(const q4hip* h, int pos) {
-  return h->list_attn != 1 || head_takes_rows(1, h->H, h->KVH, h->HD, h->kv16, pass_span(pos, 1)) ? 0 : 1;
+  return h->list_attn != 1 || head_takes_rows(1, h->H, h->KVH, h->HD, h->kv16, h->ctx, pass_span(pos, 1)) ? 0 : 1;
 }
 
 // Capture the step that takes the token at `pos`, unless it is there.
@@ -3583,9 +3580,7 @@ static int run_batch(q4hip_batch* bt, const int* first, const int* pos, int step
     HIPCHK(hipEventCreate(&e1));
     HIPCHK(hipEventRecord(e0, h->stream));
   }
-  int64_t sum = 0;
-  for (int b = 0; b < B; b++) sum += pos[b];
-  const AttnSpan sp = {*std::max_element(pos, pos + B) + steps, (int)(sum / B) + (steps + 1) / 2};
+  const AttnSpan sp = batch_span(pos, B, h->KVH, steps);
   for (int i = 0; i < steps; i++) enqueue_batch_step(bt, bt->out + (size_t)i * B, sp);
   if (ms) HIPCHK(hipEventRecord(e1, h->stream));
   HIPCHK(hipGetLastError());

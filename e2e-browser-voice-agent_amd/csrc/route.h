@@ -78,13 +78,34 @@ constexpr size_t attn_head_lds(int HD, int end) {
   return (size_t)kHeadStageBytes + (size_t)(head_row(end) + 16 + 4 * HD) * sizeof(float);
 }
 
-// The positions a call's rows look at: one past the last of any row, and a row's mean.
+// The positions a call's rows look at: one past the last of any row, and the mean of the rows on the XCD
+// that has most of them.
 struct AttnSpan {
   int end, mean;
 };
 
+// M tokens of a pass from pos on.
+constexpr AttnSpan pass_span(int pos, int M) { return {pos + M, pos + (M + 1) / 2}; }
+
 // k_attn_head's workgroups: units (row, kv head) dealt to the 8 XCDs, the G heads of a unit 8 apart.
 constexpr int attn_head_grid(int rows, int KVH, int G) { return (rows * KVH + kXcds - 1) / kXcds * kXcds * G; }
+
+// `steps` steps of B sequences at pos[]: sequences of different lengths may meet on an XCD (k_attn_head
+// deals its units from the last sequence on).
+inline AttnSpan batch_span(const int* pos, int B, int KVH, int steps) {
+  long load[kXcds] = {}, most = 0;
+  int last = 0;
+  for (int b = 0; b < B; b++) {
+    if (pos[b] > last) last = pos[b];
+    for (int g = 0; g < KVH; g++) {
+      long& l = load[((B - 1 - b) * KVH + g) % kXcds];
+      l += pos[b] + (steps + 1) / 2;
+      if (l > most) most = l;
+    }
+  }
+  const int per = (B * KVH + kXcds - 1) / kXcds;
+  return {last + steps, (int)((most + per - 1) / per)};
+}
 
 // How many of its workgroups run at once.
 constexpr int head_slots(int HD, int end) { return kCus * (attn_head_lds(HD, end) <= 80 * 1024 ? 2 : 1); }
@@ -122,23 +143,35 @@ inline bool head_takes_pass(int rows, int H, int KVH, int HD, bool kv16, AttnSpa
 //     other, and from there on the rows leave the L2 in between.  1.5B, 2 sequences of 700 2.47 / 2.39, of
 //     1,024 2.59 / 2.68; 32 of 700 2.83 / 2.75, of 3,000 4.09 / 4.83; one token of 12 layers at 700 0.71 /
 //     0.67, at 1,500 0.83 / 0.91; the smaller the group, the sooner (16 heads in groups of 4, 2 sequences of
-//     600 1.007 times as fast, of 1,024 0.94; in groups of 1 300 1.00, 1,024 0.86).  Large batches of small
-//     groups read enough on either side to hide it (groups of 4, 24 sequences of 3,000 1.05; groups of 2, 16
-//     sequences 1.05).
-//   * large groups in more workgroups than run at once: head_dim 64 past some 600 or 700 positions (0.5B,
-//     64 sequences of 500 1.92 / 1.88, of 700 2.00 / 2.06, 48 of 700 1.85 / 1.83), and past some 3,500
-//     positions, where one workgroup fits a CU (32 sequences of 3,800 83 / 91 us a layer).
-inline bool head_takes_rows(int rows, int H, int KVH, int HD, bool kv16, AttnSpan sp) {
+//     600 1.007 times as fast, of 1,024 0.94; in groups of 1 300 1.00, 1,024 0.86).  One long row is enough
+//     (16 sequences of 200 and one of 1,500 0.93 times as fast).  Large batches of small groups read enough on
+//     either side to hide it (groups of 4, 24 sequences of 3,000 1.05; groups of 2, 16 sequences 1.05).
+//   * large groups in more workgroups than run at once, where the list kernels' two workgroups fit a CU or
+//     head_dim is 64, past some 300 to 700 positions (0.5B, 64 sequences of 500 1.92 / 1.88, of 700 2.00 /
+//     2.06, 48 of 700 1.85 / 1.83; 1.5B fp16, 48 of 900 in a context of 940 0.97, of 4,352 1.09), and past some
+//     3,500 positions, where one of its own does (32 sequences of 3,800 83 / 91 us a layer).  Rows of unequal
+//     length run at once if their positions do while the longest runs (0.5B, 64 sequences of 16 to 900 1.07
+//     times as fast, of 900 0.95, every other one of 900 0.91: those meet on half the XCDs).
+inline bool head_takes_rows(int rows, int H, int KVH, int HD, bool kv16, int ctx, AttnSpan sp) {
+  if (rows == 1) sp.end = sp.mean;         // a captured step is launched for all of the context
   const int G = H / KVH, slots = head_slots(HD, sp.end), grid = attn_head_grid(rows, KVH, G);
-  const int rounds = (grid + slots - 1) / slots;
+  const long work = (long)grid * sp.mean, once = (long)slots * sp.end;
+  const bool one_round = work <= once || (4L * sp.mean <= 3L * sp.end && 4 * work <= 5 * once);
+  const bool list_pairs = 34 * 1024 + 4L * G * ctx <= 80 * 1024;       // two k_attn_pv_list workgroups fit a CU
   if (HD == 128 && !kv16) {
-    const int most = G >= 5 ? (rounds == 1 ? 832 : 640) : G >= 3 ? 704 : G == 2 ? 512 : 384;
-    const bool many = G <= 2 ? grid >= 128 * G : G == 4 && grid >= 384;
-    if (sp.mean > most && !(many && slots == 2 * kCus)) return false;
+    if (slots == 2 * kCus && 3L * sp.mean >= 2L * sp.end &&
+        (G <= 2 ? grid >= 128 * G : G == 4 && grid >= 384 && !list_pairs))
+      return true;
+    if (G >= 5 && grid > 2 * kCus && one_round) return sp.end <= 1024;
+    int most;                              // positions up to which it is the faster one
+    if (G >= 5) most = one_round ? 832 : list_pairs ? 288 : 640;
+    else most = G >= 3 ? (!one_round && list_pairs ? 400 : 704) : G == 2 ? 512 : 384;
+    if (sp.mean > most || sp.end > most + 64) return false;
   }
-  if (rounds == 1 || G <= 2) return true;
+  if (one_round || G <= 2) return true;
   if (slots == kCus) return false;
-  return HD == 128 || G <= 4 || sp.mean <= (grid <= 768 ? 704 : 576);
+  if (HD == 128) return sp.end <= 512 || !list_pairs;
+  return G == 4 || (G == 3 && !list_pairs) || sp.end <= (grid <= 768 ? 704 : 576);
 }
 
 }  // namespace q4

@@ -78,8 +78,9 @@ def test_sum_by_the_wave(name, kv):
 
 
 def test_steps_across_the_limit_of_fp32_rows():
-    """Two heads of 128 fp32 columns in one group: a token, and a small batch by its mean, takes this
-    kernel up to 512 positions and the list kernels from there (the token in two captured steps)."""
+    """Two heads of 128 fp32 columns in one group: a token, and a batch of a few sequences by its
+    longest, takes this kernel up to 512 positions and the list kernels from there (the token in two
+    captured steps)."""
     import q4hip
     shape, g, o = _pair("small128", "f32", 1000)
     try:
@@ -96,7 +97,7 @@ def test_steps_across_the_limit_of_fp32_rows():
         for i in range(14):
             assert g.forward([want[i]], 506 + i) == want[i + 1], f"token {i}"
         _same(g.read_logits(), last, "token by token")
-        lens = [505, 500, 511]                       # means of 507 (2 steps) and 520
+        lens = [505, 500, 511]                       # 512 (2 steps), then 526, in the middle
         bt = q4hip.Batch(g, 3)
         try:
             ps = [synth.prompt_ids(40 + n, n, shape.vocab) for n in lens]
